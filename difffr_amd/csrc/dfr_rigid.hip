@@ -8,119 +8,150 @@ namespace dfr {
 
 // ---------------------------------------------------------------------------
 // Pair Jacobians: TimeStepDiffDFSPH::computeRigidBodyGradient (:1226-1279) and
-// computeGradient (:1281-1482) with its helpers (:1485-1694).  One thread per
-// sample j of a dynamic, non-animated body; j walks its fluid neighbours i.
+// computeGradient (:1281-1482) with its helpers (:1485-1694).  Sixteen lanes per
+// sample j of a dynamic, non-animated body share its fluid neighbours i.
 // d(b_i)/d(v_i) = (dt) * sum_j V_j gradW_ij equals -(dt) * sum_grad_p_k_i over
 // the same neighbour set, so it is read from the factor pass instead of being
 // re-summed for every pair.
+//
+// Of a pair's 78 entries only dF/dv, dF/dx and the force depend on i; the others
+// are products of those with matrices of the sample (lever arm, omega, d(Rx0)/dq),
+// so the lanes sum 21 values over the pairs (FP64) and the products are formed
+// once per sample.  A few hundred samples with up to ~25 neighbours each leave
+// the chip idle whatever the split, so the launch costs its longest chain: one
+// thread per sample walking its list with all 78 FP64 sums took 45 us a launch
+// (1,000-particle box; 8,000: 35, 483k tank: 33), this form 6.7 (6.4, 7.1).
+// The sums over lanes and samples go through LDS in loops: straight-line shuffle
+// code of that many FP64 values is paid in instruction fetches.
 // ---------------------------------------------------------------------------
+constexpr int GL = 16;                    // lanes per sample
+constexpr int GG = DFR_BLOCK / GL;        // samples per workgroup
+constexpr int GS = 21;                    // pair sums: dF/dv (9), dF/dx (9), force (3)
 __global__ void __launch_bounds__(DFR_BLOCK)
 k_gradient(StepConst c, GradConst gc, int k_first, int k_count, int body, const uint32_t* __restrict__ dyn_idx,
            int nd, const uint32_t* __restrict__ bf, const uint32_t* __restrict__ bfcnt, const float4* __restrict__ pos,
            const float4* __restrict__ vel, const float* __restrict__ badv, const float* __restrict__ alpha,
            const float4* __restrict__ s, const float4* __restrict__ bpos, const float4* __restrict__ bvel,
            const float4* __restrict__ bx0, RigidDev* __restrict__ rig, const int* __restrict__ stop) {
+  __shared__ double part[GS][DFR_BLOCK + 1];  // + 1: the rows start in different banks
+  __shared__ double sums[GG][GS];
+  __shared__ double out[GG][78];
   // an iteration enqueued after the solve converged (device-side loop) adds nothing
   if (stop && *stop) return;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc[78];
+  const int grp = threadIdx.x / GL, lane = threadIdx.x % GL;
+  const int t = blockIdx.x * GG + grp;
+  const bool valid = t < k_count;
+  const int kk = k_first + (valid ? t : 0);
+  const uint32_t nn = valid ? bfcnt[kk] : 0u;
+  if (!__syncthreads_or(nn > 0u)) return;  // no sample of this workgroup touches the fluid
+  const uint32_t j = dyn_idx[kk];
+  const float4 bj = bpos[j];
+  const float4 vjb = bvel[j];
+  const DV3<float> xj = {bj.x, bj.y, bj.z};
+  const float Vj = bj.w;
+  const float invH = 1.f / c.dt;
+  double acc[GS];
 #pragma unroll
-  for (int k = 0; k < 78; ++k) acc[k] = 0.0;
-  if (t < k_count) {
-    const int kk = k_first + t;
-    const uint32_t j = dyn_idx[kk];
-    const float4 bj = bpos[j];
-    const float4 vjb = bvel[j];
-    const float4 x0 = bx0[j];
-    const DV3<float> xj = {bj.x, bj.y, bj.z};
-    const float Vj = bj.w;
-    const RigidDev& rb = rig[body];
-    const float qf[4] = {(float)rb.q[0], (float)rb.q[1], (float)rb.q[2], (float)rb.q[3]};
-    const DV3<float> rj = {(float)((double)bj.x - rb.x[0]), (float)((double)bj.y - rb.x[1]),
-                           (float)((double)bj.z - rb.x[2])};
-    const DV3<float> om = {(float)rb.w[0], (float)rb.w[1], (float)rb.w[2]};
-    const DM<float, 3, 4> Jq = grad_Rqp<float>(qf, DV3<float>{x0.x, x0.y, x0.z}, 1.f);
-    const DM3<float> Srj = skew(rj);
-    const float invH = 1.f / c.dt;
-    const uint32_t nn = bfcnt[kk];
-    for (uint32_t n = 0; n < nn; ++n) {
-      const uint32_t i = bf[(size_t)n * nd + kk];
-      const float bb = badv[i];
-      const float b_i = (gc.mode == 0) ? bb - 1.f : bb;
-      const float fac = alpha[i];
-      const float ki = b_i * fac * gc.coeff_trunc;  // truncated coefficient, :1266
-      const float4 pi = pos[i];
-      const float4 vi4 = vel[i];
-      const float4 si4 = s[i];
-      const float rx = pi.x - xj.x, ry = pi.y - xj.y, rz = pi.z - xj.z;
-      const float rl = sqrtf(rx * rx + ry * ry + rz * rz);
-      const float sc = cubic_gradW_scale(c.K, rl);
-      const DV3<float> gW = {sc * rx, sc * ry, sc * rz};
-      const DV3<float> gp = {-Vj * gW.x, -Vj * gW.y, -Vj * gW.z};  // grad_p_j
-      float ga, gb;
-      cubic_gradGradW_ab(c.K, rl, ga, gb);
-      DM3<float> GG = outer(DV3<float>{rx, ry, rz}, DV3<float>{rx, ry, rz}) * gb;
-      GG(0, 0) += ga; GG(1, 1) += ga; GG(2, 2) += ga;
-      const DM3<float> H = GG * Vj;  // grad2_p_j_to_xj
-      const float a = -c.dt * 1.f * ki;
-      const DV3<float> velChange = {a * gp.x, a * gp.y, a * gp.z};
-      const DV3<float> force = {-c.m_f * velChange.x * invH, -c.m_f * velChange.y * invH, -c.m_f * velChange.z * invH};
-      const DV3<float> vij = {vi4.x - vjb.x, vi4.y - vjb.y, vi4.z - vjb.z};
-      const DV3<float> GGv = mv(GG, vij);
-      DV3<float> gbx = {0.f, 0.f, 0.f}, gbv = {0.f, 0.f, 0.f}, gbvi = {0.f, 0.f, 0.f};
-      const bool on = (gc.mode == 0) ? (bb > 1.f) : (bb > 0.f);
-      if (on) {
-        if (gc.mode == 0) {
-          gbx = {-Vj * gW.x / c.rho0 - c.dt * Vj * GGv.x, -Vj * gW.y / c.rho0 - c.dt * Vj * GGv.y,
-                 -Vj * gW.z / c.rho0 - c.dt * Vj * GGv.z};
-          gbv = {-c.dt * Vj * gW.x, -c.dt * Vj * gW.y, -c.dt * Vj * gW.z};
-          gbvi = {-si4.x * c.dt, -si4.y * c.dt, -si4.z * c.dt};
-        } else {
-          gbx = {-(GGv.x * Vj), -(GGv.y * Vj), -(GGv.z * Vj)};
-          gbv = {-Vj * gW.x, -Vj * gW.y, -Vj * gW.z};
-          gbvi = {-si4.x, -si4.y, -si4.z};
-        }
-      }
-      DV3<float> gfx = {0.f, 0.f, 0.f};
-      if (fac < 0.f) {
-        const DV3<float> Hs = mv(H, DV3<float>{si4.x, si4.y, si4.z});
-        const float f2 = 2.f * fac * fac;
-        gfx = {Hs.x * f2, Hs.y * f2, Hs.z * f2};
-      }
-      const float co = gc.coeff;
-      const DV3<float> gkx = {(gbx.x * fac + gfx.x * b_i) * co, (gbx.y * fac + gfx.y * b_i) * co,
-                              (gbx.z * fac + gfx.z * b_i) * co};
-      const DM3<float> dvc_dxj = (outer(gp, gkx) + H * ki) * -1.f;
-      const DV3<float> gkv = {gbv.x * fac * co, gbv.y * fac * co, gbv.z * fac * co};
-      const DM3<float> dvc_dvj = outer(gp, gkv) * -1.f;
-      const DV3<float> gkvi = {gbvi.x * fac * co, gbvi.y * fac * co, gbvi.z * fac * co};
-      const DM3<float> dvc_dvi = outer(gp, gkvi) * -1.f;
-      const DM3<float> gFx = dvc_dxj * (-c.m_f);
-      const DM3<float> gFv = mm(inverse3(DM3<float>::eye() - dvc_dvi * c.dt), dvc_dvj * (-c.m_f));
-#pragma unroll
-      for (int k = 0; k < 9; ++k) { acc[k] += gFv.a[k]; acc[9 + k] += gFx.a[k]; }
-      if (gc.optimize_rotation) {
-        const DM<float, 3, 4> gFq = mm(gFx, Jq) + mm(mm(gFv, skew(om)), Jq);
-        const DM3<float> gFw = mm(gFv, Srj.tr());
-        const DM<float, 3, 4> gTq = mm(Srj, gFq) + mm(skew(force).tr(), Jq);
-        const DM3<float> gTw = mm(Srj, gFw);
-        const DM3<float> gTx = mm(Srj, gFx);
-        const DM3<float> gTv = mm(Srj, gFv);
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          acc[18 + k] += gFw.a[k]; acc[27 + k] += gTw.a[k]; acc[36 + k] += gTx.a[k]; acc[45 + k] += gTv.a[k];
-        }
-#pragma unroll
-        for (int k = 0; k < 12; ++k) { acc[54 + k] += gFq.a[k]; acc[66 + k] += gTq.a[k]; }
+  for (int k = 0; k < GS; ++k) acc[k] = 0.0;
+  for (uint32_t n = lane; n < nn; n += GL) {
+    const uint32_t i = bf[(size_t)n * nd + kk];
+    const float bb = badv[i];
+    const float b_i = (gc.mode == 0) ? bb - 1.f : bb;
+    const float fac = alpha[i];
+    const float ki = b_i * fac * gc.coeff_trunc;  // truncated coefficient, :1266
+    const float4 pi = pos[i];
+    const float4 vi4 = vel[i];
+    const float4 si4 = s[i];
+    const float rx = pi.x - xj.x, ry = pi.y - xj.y, rz = pi.z - xj.z;
+    const float rl = sqrtf(rx * rx + ry * ry + rz * rz);
+    const float sc = cubic_gradW_scale(c.K, rl);
+    const DV3<float> gW = {sc * rx, sc * ry, sc * rz};
+    const DV3<float> gp = {-Vj * gW.x, -Vj * gW.y, -Vj * gW.z};  // grad_p_j
+    float ga, gb;
+    cubic_gradGradW_ab(c.K, rl, ga, gb);
+    DM3<float> GG3 = outer(DV3<float>{rx, ry, rz}, DV3<float>{rx, ry, rz}) * gb;
+    GG3(0, 0) += ga; GG3(1, 1) += ga; GG3(2, 2) += ga;
+    const DM3<float> H = GG3 * Vj;  // grad2_p_j_to_xj
+    const float a = -c.dt * 1.f * ki;
+    const DV3<float> velChange = {a * gp.x, a * gp.y, a * gp.z};
+    const DV3<float> force = {-c.m_f * velChange.x * invH, -c.m_f * velChange.y * invH, -c.m_f * velChange.z * invH};
+    const DV3<float> vij = {vi4.x - vjb.x, vi4.y - vjb.y, vi4.z - vjb.z};
+    const DV3<float> GGv = mv(GG3, vij);
+    DV3<float> gbx = {0.f, 0.f, 0.f}, gbv = {0.f, 0.f, 0.f}, gbvi = {0.f, 0.f, 0.f};
+    const bool on = (gc.mode == 0) ? (bb > 1.f) : (bb > 0.f);
+    if (on) {
+      if (gc.mode == 0) {
+        gbx = {-Vj * gW.x / c.rho0 - c.dt * Vj * GGv.x, -Vj * gW.y / c.rho0 - c.dt * Vj * GGv.y,
+               -Vj * gW.z / c.rho0 - c.dt * Vj * GGv.z};
+        gbv = {-c.dt * Vj * gW.x, -c.dt * Vj * gW.y, -c.dt * Vj * gW.z};
+        gbvi = {-si4.x * c.dt, -si4.y * c.dt, -si4.z * c.dt};
+      } else {
+        gbx = {-(GGv.x * Vj), -(GGv.y * Vj), -(GGv.z * Vj)};
+        gbv = {-Vj * gW.x, -Vj * gW.y, -Vj * gW.z};
+        gbvi = {-si4.x, -si4.y, -si4.z};
       }
     }
-  }
-  const bool any = __ballot(t < k_count) != 0ull;
-  if (!any) return;
+    DV3<float> gfx = {0.f, 0.f, 0.f};
+    if (fac < 0.f) {
+      const DV3<float> Hs = mv(H, DV3<float>{si4.x, si4.y, si4.z});
+      const float f2 = 2.f * fac * fac;
+      gfx = {Hs.x * f2, Hs.y * f2, Hs.z * f2};
+    }
+    const float co = gc.coeff;
+    const DV3<float> gkx = {(gbx.x * fac + gfx.x * b_i) * co, (gbx.y * fac + gfx.y * b_i) * co,
+                            (gbx.z * fac + gfx.z * b_i) * co};
+    const DM3<float> dvc_dxj = (outer(gp, gkx) + H * ki) * -1.f;
+    const DV3<float> gkv = {gbv.x * fac * co, gbv.y * fac * co, gbv.z * fac * co};
+    const DM3<float> dvc_dvj = outer(gp, gkv) * -1.f;
+    const DV3<float> gkvi = {gbvi.x * fac * co, gbvi.y * fac * co, gbvi.z * fac * co};
+    const DM3<float> dvc_dvi = outer(gp, gkvi) * -1.f;
+    const DM3<float> gFx = dvc_dxj * (-c.m_f);
+    const DM3<float> gFv = mm(inverse3(DM3<float>::eye() - dvc_dvi * c.dt), dvc_dvj * (-c.m_f));
 #pragma unroll
-  for (int k = 0; k < 78; ++k) {
-    const double v = wave_sum_d(acc[k]);
-    if ((threadIdx.x & 63) == 0 && v != 0.0) atomicAdd(&rig[body].net[k], v);
+    for (int k = 0; k < 9; ++k) { acc[k] += gFv.a[k]; acc[9 + k] += gFx.a[k]; }
+    acc[18] += force.x; acc[19] += force.y; acc[20] += force.z;
+  }
+#pragma unroll
+  for (int k = 0; k < GS; ++k) part[k][threadIdx.x] = acc[k];
+  __syncthreads();
+  for (int k = lane; k < GS; k += GL) {
+    double v = 0.0;
+    for (int m = 0; m < GL; ++m) v += part[k][grp * GL + m];
+    sums[grp][k] = v;
+  }
+  __syncthreads();
+  if (lane == 0) {
+    const RigidDev& rb = rig[body];
+    double* o = out[grp];
+    M3d gFv, gFx;
+    for (int k = 0; k < 9; ++k) { gFv.a[k] = o[k] = sums[grp][k]; gFx.a[k] = o[9 + k] = sums[grp][9 + k]; }
+    const V3d F = {sums[grp][18], sums[grp][19], sums[grp][20]};
+    if (gc.optimize_rotation) {
+      // the sample's matrices as the reference forms them, in FP32
+      const float4 x0 = bx0[j];
+      const float qf[4] = {(float)rb.q[0], (float)rb.q[1], (float)rb.q[2], (float)rb.q[3]};
+      const DM<float, 3, 4> Jf = grad_Rqp<float>(qf, DV3<float>{x0.x, x0.y, x0.z}, 1.f);
+      M34d Jq;
+      for (int k = 0; k < 12; ++k) Jq.a[k] = (double)Jf.a[k];
+      const M3d Srj = skew(V3d{(double)(float)((double)bj.x - rb.x[0]), (double)(float)((double)bj.y - rb.x[1]),
+                               (double)(float)((double)bj.z - rb.x[2])});
+      const M3d Som = skew(V3d{(double)(float)rb.w[0], (double)(float)rb.w[1], (double)(float)rb.w[2]});
+      const M34d gFq = mm(gFx + mm(gFv, Som), Jq);
+      const M3d gFw = mm(gFv, Srj.tr());
+      const M34d gTq = mm(Srj, gFq) + mm(skew(F).tr(), Jq);
+      st3(o + 18, gFw);
+      st3(o + 27, mm(Srj, gFw));
+      st3(o + 36, mm(Srj, gFx));
+      st3(o + 45, mm(Srj, gFv));
+      for (int k = 0; k < 12; ++k) { o[54 + k] = gFq.a[k]; o[66 + k] = gTq.a[k]; }
+    }
+  }
+  __syncthreads();
+  const int k = threadIdx.x;
+  if (k < (gc.optimize_rotation ? 78 : 18)) {
+    double v = 0.0;
+    for (int m = 0; m < GG; ++m) v += out[m][k];
+    if (v != 0.0) atomicAdd(&rig[body].net[k], v);
   }
 }
 
@@ -515,7 +546,7 @@ __global__ void k_begin_step(BeginStepTable t, RigidDev* __restrict__ rig, int n
 void launch_gradient(const StepConst& c, const GradConst& gc, FluidBufs& f, BoundaryBufs& b, NbrBufs& nb,
                      RigidDev* rig, int k_first, int k_count, int body, hipStream_t s, const int* stop) {
   if (k_count <= 0) return;
-  const unsigned blocks = (unsigned)((k_count + DFR_BLOCK - 1) / DFR_BLOCK);
+  const unsigned blocks = (unsigned)((k_count + GG - 1) / GG);
   hipLaunchKernelGGL(k_gradient, dim3(blocks), dim3(DFR_BLOCK), 0, s, c, gc, k_first, k_count, body, b.dyn_idx, b.nd,
                      nb.bf, nb.bfcnt, f.pos, f.vel, f.badv, f.alpha, f.s, b.pos, b.vel, b.x0, rig, stop);
 }

@@ -1,0 +1,52 @@
+"""The reference-mode pair sums (dfr_get_net_gradients) against the oracle at
+sample counts around the kernel's groups of 16 samples a workgroup and 16
+lanes a sample: fewer, exactly and more than a group, with neighbour lists
+shorter and longer than 16, with and without the rotation entries.
+
+Tolerance: the sums hang on FP32 terms that cancel (b_i = rho* - 1), so the
+oracle's own FP32 and FP64 runs of the step differ by about 1e-3 of a block's
+largest entry; the GPU, which rounds like the FP32 run in another order, is
+held to three times the largest such spread of the blocks.
+"""
+import numpy as np
+import pytest
+
+from difffr_amd import scenes
+from difffr_amd.simulation import Simulation
+from oracle.pyoracle import OracleSim
+
+pytestmark = pytest.mark.gpu
+
+BLOCKS = [(0, 9), (9, 18), (18, 27), (27, 36), (36, 45), (45, 54), (54, 66), (66, 78)]
+
+
+@pytest.mark.parametrize("samples,rotation", [(1, 1), (15, 1), (16, 0), (17, 1), (130, 1)])
+def test_pair_sums_match_oracle(gpu_ready, samples, rotation):
+    print(f"[pair sums] {samples} samples, optimize_rotation {rotation}", flush=True)
+    sc = scenes.submerged_body(body="sphere", steps=1)
+    sc.params.update(compute_gradient=1, optimize_rotation=rotation)
+    b = sc.bodies[1]
+    b.x0 = 0.05 * scenes.fibonacci_sphere(max(samples, 2))[:samples]
+    b.x_rb = b.x_rb - np.array([0.0, 0.05, 0.0])  # deeper: lists longer than 16
+    sc.fluid_x = sc.fluid_x[np.linalg.norm(sc.fluid_x - b.x_rb, axis=1) > 0.07]
+    sc.fluid_x[:, :] = b.x_rb + 0.93 * (sc.fluid_x - b.x_rb)  # at rest density
+    sc.fluid_v = -0.5 * (sc.fluid_x - b.x_rb) / 0.07            # closing in on the body
+    g = Simulation(sc)
+    g.step(1)
+    it = g.stats()
+    ng = g.net_gradients_raw(1)
+    g.close()
+    ref = []
+    for variant in ("f32_rigid64", "f64"):
+        o = OracleSim(sc, variant)
+        o.set_fixed_iterations([it["iterations_v"]], [it["iterations"]])
+        o.step(1)
+        ref.append(o.net_gradients(1))
+    blocks = BLOCKS if rotation else BLOCKS[:2]
+    scale = [np.abs(ref[0][lo:hi]).max() for lo, hi in blocks]
+    assert min(scale) > 0.0
+    spread = max(np.abs(ref[0][lo:hi] - ref[1][lo:hi]).max() / s for (lo, hi), s in zip(blocks, scale))
+    for (lo, hi), s in zip(blocks, scale):
+        assert np.abs(ng[lo:hi] - ref[0][lo:hi]).max() <= 3.0 * spread * s, (lo, spread)
+    if not rotation:
+        assert np.all(ng[18:] == 0.0)
