@@ -24,9 +24,11 @@ constexpr int BB = PASS_BLOCK;  // build workgroup: one particle of the brick pe
 
 // Fluid neighbour slots of one particle as they are found: a 16-entry ring per
 // thread in LDS (entry e of thread t at ring[e * BB + t], so a wavefront's
-// writes are consecutive), one 16-bit write per accepted slot; whenever eight
-// are pending (a chunk of candidates adds at most 4, so at most 11 are) they
-// leave as one pack of the pack-major list.
+// writes are consecutive), one 16-bit write per candidate.  Eight pending slots
+// leave as one pack of the pack-major list; packing costs as much as testing
+// eight candidates, so the lanes of a wavefront store together, when some
+// lane's ring might not take another chunk of four (in nearly every chunk some
+// lane reaches eight).
 constexpr int RING = 16;
 struct PackWriter {
   uint16_t* ring;  // this block's ring
@@ -39,10 +41,11 @@ struct PackWriter {
   }
   // Branch-free push: the slot is written at the next free entry either way
   // (an entry past the accepted ones, which the next push overwrites; at most
-  // 11 entries are pending, so it never holds one) and counted if accepted.
-  __device__ inline void push_if(uint32_t s, bool accept) {
+  // RING - 4 are pending before a chunk, so it never holds one) and counted if
+  // d2 < h2 (compare and add with carry).
+  __device__ inline void push_if(uint32_t s, float h2, float d2) {
     ring[(n & (RING - 1)) * BB + t] = (uint16_t)s;
-    n += accept ? 1u : 0u;
+    asm("v_cmp_gt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, 0, %0, vcc" : "+v"(n) : "s"(h2), "v"(d2) : "vcc");
   }
   __device__ inline void store(uint4* __restrict__ nbr8, size_t stride, uint32_t i, uint32_t count) {
     uint32_t w[4];
@@ -59,13 +62,27 @@ struct PackWriter {
   __device__ inline void flush_full(uint4* __restrict__ nbr8, size_t stride, uint32_t i) {
     if (n - np * PACK >= (uint32_t)PACK) store(nbr8, stride, i, PACK);
   }
+  // after a chunk of up to four pushes: keeps room for the next one
+  __device__ inline void flush_chunk(uint4* __restrict__ nbr8, size_t stride, uint32_t i) {
+    if (__any(n - np * PACK > (uint32_t)(RING - 4))) flush_full(nbr8, stride, i);
+  }
   __device__ inline uint32_t finish(uint4* __restrict__ nbr8, size_t stride, uint32_t i) {
+    flush_full(nbr8, stride, i);  // at most RING - 4 pending: fewer than a pack are left
     const uint32_t rest = n - np * PACK;
     if (rest > 0u) store(nbr8, stride, i, rest);
     return n;
   }
 };
 
+// Bound by vector issue: 270 candidates a particle at rest density, walked as
+// nine rows by each lane, so a wavefront takes the longest row of its cells
+// nine times (1.6 times the mean in a packing with 8 to 27 particles a cell).
+// 13 instructions a candidate with whole chunks free of the row-end test and the
+// lanes storing together; 16, with a store in nearly every chunk, took 247 us
+// at 1M, this form 225 (483k: 144 and 132).  One cell a wavefront with the
+// candidates in the lanes and ballots for the lists: 379 us (the scalar work
+// per round of 64 outweighs the balanced lanes).
+//
 // Dynamic LDS: x, y, z of the halo in three arrays of a fixed stride, so one
 // address serves a chunk of four candidates (immediate offsets); a chunk reads
 // up to three slots past its row's end, which stay inside the arrays because
@@ -157,7 +174,8 @@ k_build_tiled(const float4* __restrict__ pos, int nf, GridDesc g, const uint32_t
       if (row == 4) r1 = self;
       if (row == 5) r0 = self + 1;
       if (in_lds) {
-        for (uint32_t s0 = r0; s0 < r1; s0 += 4) {
+        uint32_t s0 = r0;
+        auto chunk = [&](bool tail) {
           float qx[4], qy[4], qz[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
@@ -167,10 +185,15 @@ k_build_tiled(const float4* __restrict__ pos, int nf, GridDesc g, const uint32_t
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const uint32_t s = s0 + u;
-            pw.push_if(s, (s < r1) & (dist2_exact(p.x, p.y, p.z, qx[u], qy[u], qz[u]) < h2));
+            float d2 = dist2_exact(p.x, p.y, p.z, qx[u], qy[u], qz[u]);
+            if (tail && u > 0 && s >= r1) d2 = h2;  // past the row's end
+            pw.push_if(s, h2, d2);
           }
-          pw.flush_full(nbr8, stride, i);
-        }
+          pw.flush_chunk(nbr8, stride, i);
+        };
+        // whole chunks need no test for the row's end
+        for (; s0 + 4u <= r1; s0 += 4) chunk(false);
+        if (s0 < r1) chunk(true);
       } else {
         for (uint32_t s = r0; s < r1; ++s) {
           const float4 q = pos[tile_global<BB>(T, s)];
