@@ -70,7 +70,7 @@ __device__ inline void atomic_add3(double* p, float x, float y, float z) {
 // vbar is the adjoint of the updated velocity (unchanged: the update adds to v).
 // LDS per slot: x, y, z, vbar (3), k.
 // ---------------------------------------------------------------------------
-template <int MODE>
+template <int MODE, int L>
 __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(6, 8)))
 k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict__ vbar,
                const float* kacc, float kacc_scale, const float* __restrict__ bval,
@@ -79,10 +79,9 @@ k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict_
   __shared__ TileHdr<RB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   BrickView B;
-  if (!brick_open<RB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<RB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;        // x, y, z, k
@@ -90,7 +89,7 @@ k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict_
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[PTR];
-    map_indices<RB>(a.tmap, brick, total, js);
+    map_indices<RB>(a.tmap, B.brick, total, js);
     float4 q[PTR], w[PTR];
     float kk[PTR];
 #pragma unroll
@@ -107,7 +106,8 @@ k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict_
   }
   __syncthreads();
   const size_t stride = (size_t)c.nf;
-  for (uint32_t i = B.own_begin + t; i < B.own_end; i += RB) {
+  const int l = t % L;  // lane of the particle
+  for (uint32_t i = B.own_begin + t / L; i < B.own_end; i += RB / L) {
     const float ki = k[i];
     const float4 p = a.x[i];
     const float4 vb = vbar[i];
@@ -129,24 +129,24 @@ k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict_
       xfz = fmaf(a, uz, fmaf(b, rz, xfz));
     };
     if (in_lds) {
-      for_fluid_groups<2>(a.nbr8, stride, i, nF, [&](uint32_t s) { return Slot8{LA[s], LB[s]}; },
-                          [&](const Slot8& q, bool live) {
-                            pair(q.a.x, q.a.y, q.a.z, q.b.x, q.b.y, q.b.z, q.a.w, live);
-                          });
+      for_fluid_lanes<2, L>(a.nbr8, stride, i, nF, l, [&](uint32_t s) { return Slot8{LA[s], LB[s]}; },
+                            [&](const Slot8& q, bool live) {
+                              pair(q.a.x, q.a.y, q.a.z, q.b.x, q.b.y, q.b.z, q.a.w, live);
+                            });
     } else {
-      for_fluid_slots_rolled(a.nbr8, stride, i, nF, [&](uint32_t s) {
+      for_fluid_slots_rolled<L>(a.nbr8, stride, i, nF, [&](uint32_t s) {
         const uint32_t j = tile_global<RB>(T, s);
         const float4 q = a.x[j];
         const float4 w = vbar[j];
         pair(q.x, q.y, q.z, w.x, w.y, w.z, k[j], true);
-      });
+      }, l);
     }
     const float dtVf = c.dt * c.V_f;
     float kb = dtVf * kbf;
     float xbx = dtVf * xfx, xby = dtVf * xfy, xbz = dtVf * xfz;
     if (fabsf(ki) > c.eps) {
       auto load = [&](uint32_t j) { return a.bx[j]; };
-      for_boundary_groups<2>(a.nbrB, stride, i, nB, load, [&](const float4& q, uint32_t j) {
+      for_boundary_groups<2, L>(a.nbrB, stride, i, nB, load, [&](const float4& q, uint32_t j, uint32_t) {
         const float Vb = q.w;
         const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
         const PairCE ce = cubic_ce(c.K, rx * rx + ry * ry + rz * rz);
@@ -178,8 +178,10 @@ k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict_
           sx += fy * Tz - fz * Ty; sy += fz * Tx - fx * Tz; sz += fx * Ty - fy * Tx;
           atomic_add3(a.sxb + 3 * (size_t)sd, sx, sy, sz);
         }
-      });
+      }, l);
     }
+    kb = lane_sum<L>(kb); xbx = lane_sum<L>(xbx); xby = lane_sum<L>(xby); xbz = lane_sum<L>(xbz);
+    if (l != 0) continue;
     if (kacc) kb += kacc_scale * kacc[i];
     float4 xo = xbar[i];
     xo.x += xbx; xo.y += xby; xo.z += xbz;
@@ -217,16 +219,16 @@ k_adj_update_t(AdjPass a, const float* __restrict__ k, const float4* __restrict_
 //   xbar_i += V_f sum_j (d_i + d_j) H_ij (v_i - v_j) + d_i sum_b V_b H_ib (v_i - v_b)
 // LDS per slot: x, y, z, v (3), d.
 // ---------------------------------------------------------------------------
+template <int L>
 __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(6, 8)))
 k_adj_delta_t(AdjPass a, const float4* __restrict__ v, const float* __restrict__ dbar, float4* __restrict__ vbar,
               float4* __restrict__ xbar) {
   __shared__ TileHdr<RB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   BrickView B;
-  if (!brick_open<RB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<RB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;        // x, y, z, dbar
@@ -234,7 +236,7 @@ k_adj_delta_t(AdjPass a, const float4* __restrict__ v, const float* __restrict__
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[PTR];
-    map_indices<RB>(a.tmap, brick, total, js);
+    map_indices<RB>(a.tmap, B.brick, total, js);
     float4 q[PTR], w[PTR];
     float dd[PTR];
 #pragma unroll
@@ -251,7 +253,8 @@ k_adj_delta_t(AdjPass a, const float4* __restrict__ v, const float* __restrict__
   }
   __syncthreads();
   const size_t stride = (size_t)c.nf;
-  for (uint32_t i = B.own_begin + t; i < B.own_end; i += RB) {
+  const int l = t % L;  // lane of the particle
+  for (uint32_t i = B.own_begin + t / L; i < B.own_end; i += RB / L) {
     const float di = dbar[i];
     const float4 p = a.x[i];
     const float4 vi = v[i];
@@ -270,23 +273,23 @@ k_adj_delta_t(AdjPass a, const float4* __restrict__ v, const float* __restrict__
       hx += sc * ux + se * rx; hy += sc * uy + se * ry; hz += sc * uz + se * rz;
     };
     if (in_lds) {
-      for_fluid_groups<2>(a.nbr8, stride, i, nF, [&](uint32_t s) { return Slot8{LA[s], LB[s]}; },
-                          [&](const Slot8& q, bool live) {
-                            pair(q.a.x, q.a.y, q.a.z, q.b.x, q.b.y, q.b.z, q.a.w, live);
-                          });
+      for_fluid_lanes<2, L>(a.nbr8, stride, i, nF, l, [&](uint32_t s) { return Slot8{LA[s], LB[s]}; },
+                            [&](const Slot8& q, bool live) {
+                              pair(q.a.x, q.a.y, q.a.z, q.b.x, q.b.y, q.b.z, q.a.w, live);
+                            });
     } else {
-      for_fluid_slots_rolled(a.nbr8, stride, i, nF, [&](uint32_t s) {
+      for_fluid_slots_rolled<L>(a.nbr8, stride, i, nF, [&](uint32_t s) {
         const uint32_t j = tile_global<RB>(T, s);
         const float4 q = a.x[j];
         const float4 w = v[j];
         pair(q.x, q.y, q.z, w.x, w.y, w.z, dbar[j], true);
-      });
+      }, l);
     }
     float vbx = c.V_f * gx, vby = c.V_f * gy, vbz = c.V_f * gz;
     float xbx = c.V_f * hx, xby = c.V_f * hy, xbz = c.V_f * hz;
     if (di != 0.f) {
       auto load = [&](uint32_t j) { return Slot8{a.bx[j], a.bv[j]}; };
-      for_boundary_groups<2>(a.nbrB, stride, i, nB, load, [&](const Slot8& s8, uint32_t j) {
+      for_boundary_groups<2, L>(a.nbrB, stride, i, nB, load, [&](const Slot8& s8, uint32_t j, uint32_t) {
         const float4 q = s8.a, vbj = s8.b;
         const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
         const PairCE ce = cubic_ce(c.K, rx * rx + ry * ry + rz * rz);
@@ -302,8 +305,11 @@ k_adj_delta_t(AdjPass a, const float4* __restrict__ v, const float* __restrict__
           atomic_add3(a.svb + 3 * (size_t)sd, -gbx, -gby, -gbz);
           atomic_add3(a.sxb + 3 * (size_t)sd, -tbx, -tby, -tbz);
         }
-      });
+      }, l);
     }
+    vbx = lane_sum<L>(vbx); vby = lane_sum<L>(vby); vbz = lane_sum<L>(vbz);
+    xbx = lane_sum<L>(xbx); xby = lane_sum<L>(xby); xbz = lane_sum<L>(xbz);
+    if (l != 0) continue;
     float4 vo = vbar[i];
     vo.x += vbx; vo.y += vby; vo.z += vbz;
     vbar[i] = vo;
@@ -323,6 +329,7 @@ k_adj_delta_t(AdjPass a, const float4* __restrict__ v, const float* __restrict__
 //           - 2 Sb_i sum_b V_b H_ib G_i
 // LDS per slot: x, y, z, Sb, rb, G (3).
 // ---------------------------------------------------------------------------
+template <int L>
 __global__ void __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(2, 8)))
 k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restrict__ alpha_bar,
                const float* __restrict__ rho_bar, const float4* __restrict__ G, float4* __restrict__ xbar,
@@ -330,10 +337,9 @@ k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restri
   __shared__ TileHdr<RB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   BrickView B;
-  if (!brick_open<RB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<RB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;        // x, y, z, Sb
@@ -342,7 +348,7 @@ k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restri
   auto sbar = [&](uint32_t j) { const float al = alpha[j]; return alpha_bar[j] * al * al; };
   if (in_lds) {
     uint32_t js[PTR];
-    map_indices<RB>(a.tmap, brick, total, js);
+    map_indices<RB>(a.tmap, B.brick, total, js);
     float4 q[PTR], g[PTR];
     float sb[PTR], rb[PTR];
 #pragma unroll
@@ -359,7 +365,8 @@ k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restri
   }
   __syncthreads();
   const size_t stride = (size_t)c.nf;
-  for (uint32_t i = B.own_begin + t; i < B.own_end; i += RB) {
+  const int l = t % L;  // lane of the particle
+  for (uint32_t i = B.own_begin + t / L; i < B.own_end; i += RB / L) {
     const float Si = sbar(i), ri = rho_bar[i];
     const float4 p = a.x[i];
     const float4 Gi = G[i];
@@ -381,17 +388,17 @@ k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restri
       fx += ce.c * ux + er * rx; fy += ce.c * uy + er * ry; fz += ce.c * uz + er * rz;
     };
     if (in_lds) {
-      for_fluid_groups<2>(a.nbr8, stride, i, nF, [&](uint32_t s) { return Slot8{LA[s], LB[s]}; },
-                          [&](const Slot8& q, bool live) {
-                            pair(q.a.x, q.a.y, q.a.z, q.a.w, q.b.x, q.b.y, q.b.z, q.b.w, live);
-                          });
+      for_fluid_lanes<2, L>(a.nbr8, stride, i, nF, l, [&](uint32_t s) { return Slot8{LA[s], LB[s]}; },
+                            [&](const Slot8& q, bool live) {
+                              pair(q.a.x, q.a.y, q.a.z, q.a.w, q.b.x, q.b.y, q.b.z, q.b.w, live);
+                            });
     } else {
-      for_fluid_slots_rolled(a.nbr8, stride, i, nF, [&](uint32_t s) {
+      for_fluid_slots_rolled<L>(a.nbr8, stride, i, nF, [&](uint32_t s) {
         const uint32_t j = tile_global<RB>(T, s);
         const float4 q = a.x[j];
         const float4 g = G[j];
         pair(q.x, q.y, q.z, sbar(j), rho_bar[j], g.x, g.y, g.z, true);
-      });
+      }, l);
     }
     const float tv = 2.f * c.V_f;
     float xbx = c.V_f * dx + tv * fx, xby = c.V_f * dy + tv * fy, xbz = c.V_f * dz + tv * fz;
@@ -399,7 +406,7 @@ k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restri
     const float rib = ri + (rbb ? rbb[i] : 0.f);
     if (Si != 0.f || rib != 0.f) {
       auto load = [&](uint32_t j) { return a.bx[j]; };
-      for_boundary_groups<2>(a.nbrB, stride, i, nB, load, [&](const float4& q, uint32_t j) {
+      for_boundary_groups<2, L>(a.nbrB, stride, i, nB, load, [&](const float4& q, uint32_t j, uint32_t) {
         const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
         const PairCE ce = cubic_ce(c.K, rx * rx + ry * ry + rz * rz);
         const float sr = rib * q.w * ce.c;
@@ -410,8 +417,10 @@ k_adj_factor_t(AdjPass a, const float* __restrict__ alpha, const float* __restri
         const float tx = sr * rx - hx, ty = sr * ry - hy, tz = sr * rz - hz;
         xbx += tx; xby += ty; xbz += tz;
         if ((int)j >= a.nb_static) atomic_add3(a.sxb + 3 * (size_t)(j - (uint32_t)a.nb_static), -tx, -ty, -tz);
-      });
+      }, l);
     }
+    xbx = lane_sum<L>(xbx); xby = lane_sum<L>(xby); xbz = lane_sum<L>(xbz);
+    if (l != 0) continue;
     float4 xo = xbar[i];
     xo.x += xbx; xo.y += xby; xo.z += xbz;
     xbar[i] = xo;
@@ -601,36 +610,26 @@ static inline unsigned nblk(size_t n) { return (unsigned)((n + DFR_BLOCK - 1) / 
 // dynamic LDS of the reverse passes: two 16-byte records per staged halo slot
 static inline size_t shm_slots(const AdjPass& a, int floats) { return sizeof(float) * (size_t)a.cap * floats; }
 
+// The kernel of a mode, for one or four lanes per particle.
+using AdjUpdateKernel = decltype(&k_adj_update_t<0, 1>);
+static AdjUpdateKernel adj_update_kernel(int mode, bool four) {
+  switch (mode) {
+    case ADJ_DIV_ITER: return four ? k_adj_update_t<ADJ_DIV_ITER, 4> : k_adj_update_t<ADJ_DIV_ITER, 1>;
+    case ADJ_PRESSURE_ITER: return four ? k_adj_update_t<ADJ_PRESSURE_ITER, 4> : k_adj_update_t<ADJ_PRESSURE_ITER, 1>;
+    case ADJ_DIV_WARM: return four ? k_adj_update_t<ADJ_DIV_WARM, 4> : k_adj_update_t<ADJ_DIV_WARM, 1>;
+    case ADJ_PRESSURE_WARM: return four ? k_adj_update_t<ADJ_PRESSURE_WARM, 4> : k_adj_update_t<ADJ_PRESSURE_WARM, 1>;
+    case ADJ_DIV_WARM_LEARNED:
+      return four ? k_adj_update_t<ADJ_DIV_WARM_LEARNED, 4> : k_adj_update_t<ADJ_DIV_WARM_LEARNED, 1>;
+    default: return four ? k_adj_update_t<ADJ_PRESSURE_WARM_LEARNED, 4> : k_adj_update_t<ADJ_PRESSURE_WARM_LEARNED, 1>;
+  }
+}
+
 void launch_adj_update(const AdjPass& a, int mode, const float* k, const float4* vbar, const float* kacc,
                        float kacc_scale, const float* bval, const float* kprev, const float* alpha, float* out,
                        float* alpha_bar, float* rho_bar, float4* xbar, hipStream_t s) {
-  const dim3 grid(nbricks(a.g)), blk(RB);
-  const size_t SHM8 = shm_slots(a, 8);
-  switch (mode) {
-    case ADJ_DIV_ITER:
-      hipLaunchKernelGGL(k_adj_update_t<ADJ_DIV_ITER>, grid, blk, SHM8, s, a, k, vbar, kacc, kacc_scale, bval, kprev,
-                         alpha, out, alpha_bar, rho_bar, xbar);
-      break;
-    case ADJ_PRESSURE_ITER:
-      hipLaunchKernelGGL(k_adj_update_t<ADJ_PRESSURE_ITER>, grid, blk, SHM8, s, a, k, vbar, kacc, kacc_scale, bval,
-                         kprev, alpha, out, alpha_bar, rho_bar, xbar);
-      break;
-    case ADJ_DIV_WARM:
-      hipLaunchKernelGGL(k_adj_update_t<ADJ_DIV_WARM>, grid, blk, SHM8, s, a, k, vbar, kacc, kacc_scale, bval, kprev,
-                         alpha, out, alpha_bar, rho_bar, xbar);
-      break;
-    case ADJ_PRESSURE_WARM:
-      hipLaunchKernelGGL(k_adj_update_t<ADJ_PRESSURE_WARM>, grid, blk, SHM8, s, a, k, vbar, kacc, kacc_scale, bval,
-                         kprev, alpha, out, alpha_bar, rho_bar, xbar);
-      break;
-    case ADJ_DIV_WARM_LEARNED:
-      hipLaunchKernelGGL(k_adj_update_t<ADJ_DIV_WARM_LEARNED>, grid, blk, SHM8, s, a, k, vbar, kacc, kacc_scale, bval,
-                         kprev, alpha, out, alpha_bar, rho_bar, xbar);
-      break;
-    default:
-      hipLaunchKernelGGL(k_adj_update_t<ADJ_PRESSURE_WARM_LEARNED>, grid, blk, SHM8, s, a, k, vbar, kacc, kacc_scale,
-                         bval, kprev, alpha, out, alpha_bar, rho_bar, xbar);
-  }
+  hipLaunchKernelGGL(adj_update_kernel(mode, a.parts_log2 > 0), dim3(pass_grid(a.g, a.parts_log2)), dim3(RB),
+                     shm_slots(a, 8), s, a, k, vbar, kacc, kacc_scale, bval, kprev, alpha, out, alpha_bar, rho_bar,
+                     xbar);
 }
 
 // ---------------------------------------------------------------------------
@@ -656,10 +655,9 @@ k_adj_viscosity_t(AdjPass a, const float4* __restrict__ v, const float* __restri
   __shared__ TileHdr<RB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   BrickView B;
-  if (!brick_open<RB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<RB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;
@@ -668,7 +666,7 @@ k_adj_viscosity_t(AdjPass a, const float4* __restrict__ v, const float* __restri
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[PTR];
-    map_indices<RB>(a.tmap, brick, total, js);
+    map_indices<RB>(a.tmap, B.brick, total, js);
     float4 q[PTR], w[PTR], ab[PTR];
     float rr[PTR];
 #pragma unroll
@@ -758,13 +756,16 @@ __global__ void k_adj_scale4(int n, float dt, const float4* __restrict__ vbar, f
 
 void launch_adj_delta(const AdjPass& a, const float4* v, const float* dbar, float4* vbar, float4* xbar,
                       hipStream_t s) {
-  hipLaunchKernelGGL(k_adj_delta_t, dim3(nbricks(a.g)), dim3(RB), shm_slots(a, 8), s, a, v, dbar, vbar, xbar);
+  hipLaunchKernelGGL(a.parts_log2 > 0 ? k_adj_delta_t<4> : k_adj_delta_t<1>, dim3(pass_grid(a.g, a.parts_log2)),
+                     dim3(RB), shm_slots(a, 8), s, a, v, dbar, vbar, xbar);
 }
 
-void launch_adj_viscosity(const AdjPass& a, int mode, const float4* v, const float* rho, const float4* vbar_in,
+void launch_adj_viscosity(const AdjPass& pass, int mode, const float4* v, const float* rho, const float4* vbar_in,
                           float4* abar, const ForceConst& fc, float4* vbar, float4* xbar, float* rho_bar,
                           hipStream_t s) {
-  if (a.c.nf <= 0) return;
+  if (pass.c.nf <= 0) return;
+  AdjPass a = pass;
+  a.parts_log2 = 0;  // once a step: one workgroup per brick at every size
   hipLaunchKernelGGL(k_adj_scale4, dim3(nblk(a.c.nf)), dim3(DFR_BLOCK), 0, s, a.c.nf, a.c.dt, vbar_in, abar);
   const size_t shm = (2 * sizeof(float4) + sizeof(float2)) * (size_t)a.cap;
   if (mode == 1)
@@ -777,8 +778,8 @@ void launch_adj_viscosity(const AdjPass& a, int mode, const float4* v, const flo
 
 void launch_adj_factor(const AdjPass& a, const float* alpha, const float* alpha_bar, const float* rho_bar,
                        const float4* G, float4* xbar, const float* rbb, hipStream_t s) {
-  hipLaunchKernelGGL(k_adj_factor_t, dim3(nbricks(a.g)), dim3(RB), shm_slots(a, 8), s, a, alpha, alpha_bar, rho_bar, G,
-                     xbar, rbb);
+  hipLaunchKernelGGL(a.parts_log2 > 0 ? k_adj_factor_t<4> : k_adj_factor_t<1>, dim3(pass_grid(a.g, a.parts_log2)),
+                     dim3(RB), shm_slots(a, 8), s, a, alpha, alpha_bar, rho_bar, G, xbar, rbb);
 }
 
 void launch_adj_position(int n, float dt, const float4* xbar, float4* vbar, hipStream_t s) {
@@ -809,18 +810,13 @@ void set_adjoint_kernel_attributes() {
   (void)hipFuncSetAttribute((const void*)k_adj_viscosity_t<1>, hipFuncAttributeMaxDynamicSharedMemorySize, s10);
   (void)hipFuncSetAttribute((const void*)k_adj_viscosity_t<2>, hipFuncAttributeMaxDynamicSharedMemorySize, s10);
   const int s8 = (int)(sizeof(float) * TILE_CAP * 8);
-  (void)hipFuncSetAttribute((const void*)k_adj_update_t<ADJ_DIV_ITER>, hipFuncAttributeMaxDynamicSharedMemorySize, s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_update_t<ADJ_PRESSURE_ITER>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_update_t<ADJ_DIV_WARM>, hipFuncAttributeMaxDynamicSharedMemorySize, s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_update_t<ADJ_PRESSURE_WARM>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_update_t<ADJ_DIV_WARM_LEARNED>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_update_t<ADJ_PRESSURE_WARM_LEARNED>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_delta_t, hipFuncAttributeMaxDynamicSharedMemorySize, s8);
-  (void)hipFuncSetAttribute((const void*)k_adj_factor_t, hipFuncAttributeMaxDynamicSharedMemorySize, s8);
+  for (int mode = ADJ_DIV_ITER; mode <= ADJ_PRESSURE_WARM_LEARNED; ++mode)
+    for (bool four : {false, true})
+      (void)hipFuncSetAttribute((const void*)adj_update_kernel(mode, four), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                s8);
+  for (const void* k : {(const void*)k_adj_delta_t<1>, (const void*)k_adj_delta_t<4>, (const void*)k_adj_factor_t<1>,
+                        (const void*)k_adj_factor_t<4>})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, s8);
 }
 
 }  // namespace dfr

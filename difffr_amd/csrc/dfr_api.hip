@@ -247,7 +247,7 @@ struct dfr_ctx {
   // (divergence, pressure), per-iteration probes in mapped pinned memory,
   // and two events the host waits on one iteration late
   int* d_stop = nullptr;
-  double* d_part = nullptr;          // per-brick residual partials of the current recompute launch
+  double* d_part = nullptr;          // per-workgroup residual partials of the current recompute launch
   int nparts = 0;
   SolveProbe* h_probe = nullptr;
   SolveProbe* d_probe = nullptr;
@@ -1199,6 +1199,7 @@ void reverse_step(dfr_ctx* c, const StepTapeDev& T) {
   a.nbr8 = T.nbr8; a.thdr = T.thdr; a.tmap = T.tmap; a.nbrB = T.nbrB; a.cnt = T.cnt;
   a.bx = T.bpos; a.bv = T.bvel; a.bx0 = c->b.x0; a.nb_static = c->b.n - c->b.nd;
   a.cap = c->nb.cap;
+  a.parts_log2 = c->nb.parts_log2;
   a.sxb = A.sxb; a.svb = A.svb; a.body = A.body;
   {
     Timed t(c, TC_ADJ_MISC);
@@ -1792,7 +1793,8 @@ int dfr_init(dfr_ctx* c) {
     HIPCHK(hipHostMalloc((void**)&c->h_overflow, sizeof(uint32_t) * 4, hipHostMallocDefault));
     c->h_overflow[0] = c->h_overflow[1] = c->h_overflow[2] = c->h_overflow[3] = 0;
     c->d_stop = dalloc<int>(c, 2);
-    c->nparts = (int)(c->grid.bn[0] * c->grid.bn[1] * c->grid.bn[2]);
+    c->nb.parts_log2 = gather_parts_log2(nf);
+    c->nparts = (int)(c->grid.bn[0] * c->grid.bn[1] * c->grid.bn[2]) << c->nb.parts_log2;
     c->d_part = dalloc<double>(c, c->nparts);
     c->probe_cap = std::max(c->P.max_iterations, c->P.max_iterations_v) + 1;
     HIPCHK(hipHostMalloc((void**)&c->h_probe, sizeof(SolveProbe) * 2 * c->probe_cap,

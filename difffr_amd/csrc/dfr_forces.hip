@@ -53,16 +53,15 @@ k_normals_t(PassArgs a, const float* __restrict__ rho, float4* __restrict__ nrm)
   __shared__ TileHdr<FB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   BrickView B;
-  if (!brick_open<FB>(a.g, a.fstart, a.thdr, brick, a.cap, T, B)) return;
+  if (!brick_open<FB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[FT];
-    map_indices<FB>(a.tmap, brick, total, js);
+    map_indices<FB>(a.tmap, B.brick, total, js);
     float4 q[FT];
     float rr[FT];
 #pragma unroll
@@ -108,9 +107,8 @@ k_he_color_t(PassArgs a, const float* __restrict__ rho, const float* __restrict_
   __shared__ TileHdr<FB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   BrickView B;
-  if (!brick_open<FB>(a.g, a.fstart, a.thdr, brick, a.cap, T, B)) return;
+  if (!brick_open<FB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;
@@ -118,7 +116,7 @@ k_he_color_t(PassArgs a, const float* __restrict__ rho, const float* __restrict_
   auto weight = [&](uint32_t j) { return PASS == 0 ? c.m_f / rho[j] : (c.m_f / rho[j]) * color[j]; };
   if (in_lds) {
     uint32_t js[FT];
-    map_indices<FB>(a.tmap, brick, total, js);
+    map_indices<FB>(a.tmap, B.brick, total, js);
     float4 q[FT];
     float ww[FT];
 #pragma unroll
@@ -162,7 +160,7 @@ k_he_color_t(PassArgs a, const float* __restrict__ rho, const float* __restrict_
     if (PASS == 0) {
       float sb = 0.f;
       for_boundary_groups(a.nbrB, stride, i, nB, [&](uint32_t j) { return a.bpos[j]; },
-                          [&](const float4& q, uint32_t) {
+                          [&](const float4& q, uint32_t, uint32_t) {
                             const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
                             sb += q.w * cubic_W(c.K, sqrtf(rx * rx + ry * ry + rz * rz));
                           });
@@ -183,10 +181,9 @@ k_forces_t(PassArgs a, const float* __restrict__ rho, const float4* __restrict__
   __shared__ TileHdr<FB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   BrickView B;
-  if (!brick_open<FB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<FB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;
@@ -195,7 +192,7 @@ k_forces_t(PassArgs a, const float* __restrict__ rho, const float4* __restrict__
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[FT];
-    map_indices<FB>(a.tmap, brick, total, js);
+    map_indices<FB>(a.tmap, B.brick, total, js);
     float4 q[FT], v[FT], n[FT];
     float rr[FT];
 #pragma unroll
@@ -287,7 +284,7 @@ k_forces_t(PassArgs a, const float* __restrict__ rho, const float4* __restrict__
     if (he && f.st_kb != 0.f) {
       const float hb = 0.25f * f.st_kb / ri * ni.x;  // kb gradC2_i / (4 rho_i)
       for_boundary_groups(a.nbrB, stride, i, nB, [&](uint32_t j) { return a.bpos[j]; },
-                          [&](const float4& q, uint32_t j) {
+                          [&](const float4& q, uint32_t j, uint32_t) {
                             const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
                             const float s = hb * q.w * cubic_grad_c(c.K, rx * rx + ry * ry + rz * rz);
                             const float ax = s * rx, ay = s * ry, az = s * rz;
@@ -314,7 +311,7 @@ k_forces_t(PassArgs a, const float* __restrict__ rho, const float4* __restrict__
     }
     if (f.st_method == 2 && f.st_kb != 0.f) {
       for_boundary_groups(a.nbrB, stride, i, nB, [&](uint32_t j) { return a.bpos[j]; },
-                          [&](const float4& q, uint32_t) {
+                          [&](const float4& q, uint32_t, uint32_t) {
                             const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
                             const float r2 = rx * rx + ry * ry + rz * rz;
                             if (r2 > 1.0e-9f) {
@@ -394,12 +391,12 @@ __global__ void k_set_u32(uint32_t* __restrict__ p, uint32_t v) { *p = v; }
 void launch_normals_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidBufs& f, BoundaryBufs& b,
                       NbrBufs& nb, float4* nrm, hipStream_t s) {
   hipLaunchKernelGGL(k_normals_t, dim3(nbricks(g)), dim3(FB), sizeof(float4) * (size_t)nb.cap, s,
-                     make_args(c, g, gb, f, b, nb), f.rho, nrm);
+                     whole_bricks(make_args(c, g, gb, f, b, nb)), f.rho, nrm);
 }
 
 void launch_he_color_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidBufs& f, BoundaryBufs& b,
                        NbrBufs& nb, float* color, float* gc2, hipStream_t s) {
-  const PassArgs a = make_args(c, g, gb, f, b, nb);
+  const PassArgs a = whole_bricks(make_args(c, g, gb, f, b, nb));
   const size_t shm = sizeof(float4) * (size_t)nb.cap;
   hipLaunchKernelGGL(k_he_color_t<0>, dim3(nbricks(g)), dim3(FB), shm, s, a, f.rho, nullptr, color);
   hipLaunchKernelGGL(k_he_color_t<1>, dim3(nbricks(g)), dim3(FB), shm, s, a, f.rho, color, gc2);
@@ -409,7 +406,7 @@ void launch_forces_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidB
                      NbrBufs& nb, const float4* nrm, const float* gc2, float4* acc, RigidDev* rig,
                      const ForceConst& fc, hipStream_t s) {
   const size_t shm = (2 * sizeof(float4) + sizeof(float2)) * (size_t)nb.cap;
-  hipLaunchKernelGGL(k_forces_t, dim3(nbricks(g)), dim3(FB), shm, s, make_args(c, g, gb, f, b, nb), f.rho, nrm, gc2,
+  hipLaunchKernelGGL(k_forces_t, dim3(nbricks(g)), dim3(FB), shm, s, whole_bricks(make_args(c, g, gb, f, b, nb)), f.rho, nrm, gc2,
                      acc, rig, fc);
 }
 

@@ -110,6 +110,7 @@ struct PassArgs {
   const uint32_t* cnt;
   int nb_static;
   int cap;  // halo slots staged in LDS (larger halos read global memory)
+  int parts_log2;  // workgroups per brick: 2^parts_log2 (NbrBufs)
 };
 
 inline unsigned nbricks(const GridDesc& g) { return (unsigned)(g.bn[0] * g.bn[1] * g.bn[2]); }
@@ -121,27 +122,42 @@ inline PassArgs make_args(const StepConst& c, const GridDesc& g, GridBufs& gb, F
   a.bx0 = b.x0; a.nbr8 = nb.nbr8; a.nbrB = nb.nbrB; a.cnt = nb.cnt; a.nb_static = b.n - b.nd;
   a.thdr = nb.thdr; a.tmap = nb.tmap;
   a.cap = nb.cap;
+  a.parts_log2 = nb.parts_log2;
   return a;
 }
 
-// A pass's view of its brick.  The build leaves, per brick, a header (own
-// particle range, halo total) and the halo's slot -> particle map, so a pass
+// The passes that run once a step: one workgroup per brick at every size.
+inline PassArgs whole_bricks(PassArgs a) {
+  a.parts_log2 = 0;
+  return a;
+}
+// Workgroups of a gather pass.
+inline unsigned pass_grid(const GridDesc& g, int parts_log2) { return nbricks(g) << parts_log2; }
+
+// A pass's view of its brick: the particles of its own that this workgroup
+// handles (all of them, or one of 2^parts_log2 ranges of whole wavefronts of
+// four lanes a particle; each stages the whole halo).  The build leaves, per
+// brick, a header (own particle range, halo total) and the halo's slot -> particle map, so a pass
 // starts with one header load and coalesced map loads; only a halo beyond the
 // LDS capacity sets up the cell table for the binary-search fallback.
 struct BrickView {
   uint32_t own_begin, own_end, total;
+  uint32_t brick, block;  // block: this workgroup's number in the pass
   bool in_lds;
 };
-template <int NT>
-__device__ inline bool brick_open(const GridDesc& g, const uint32_t* __restrict__ fstart, const uint4* __restrict__ thdr,
-                                  uint32_t brick, int cap, TileHdr<NT>& T, BrickView& B) {
-  const uint4 h = thdr[brick];
-  if (h.x == h.y) return false;  // no own particle (uniform exit)
-  B.own_begin = h.x;
-  B.own_end = h.y;
+template <int NT, class Args>
+__device__ inline bool brick_open(const Args& a, TileHdr<NT>& T, BrickView& B) {
+  B.block = xcd_block();
+  B.brick = B.block >> a.parts_log2;
+  const uint4 h = a.thdr[B.brick];
+  const uint32_t parts = 1u << a.parts_log2, part = B.block & (parts - 1u);
+  const uint32_t per = (((h.y - h.x + parts - 1u) >> a.parts_log2) + 15u) & ~15u;
+  B.own_begin = h.x + (parts > 1u ? part * per : 0u);
+  B.own_end = parts > 1u ? min(B.own_begin + per, h.y) : h.y;
+  if (B.own_begin >= B.own_end) return false;  // no own particle (uniform exit)
   B.total = h.z;
-  B.in_lds = h.z <= (uint32_t)cap;
-  if (!B.in_lds) tile_setup<NT>(g, fstart, brick, T);
+  B.in_lds = h.z <= (uint32_t)a.cap;
+  if (!B.in_lds) tile_setup<NT>(a.g, a.fstart, B.brick, T);
   return true;
 }
 template <int NT, int CAP = TILE_CAP>
@@ -210,24 +226,156 @@ __device__ inline void for_fluid_groups(const uint4* __restrict__ nbr8, size_t s
   }
 }
 
+// The same with four lanes per particle, for the reverse passes (see
+// gather_parts_log2): lane l takes the slots 2 l and 2 l + 1 of each pack, two
+// packs a round; the partial sums of the lanes are added at the end (lane_sum).
+template <int G, int L, class Load, class Body>
+__device__ inline void for_fluid_lanes(const uint4* __restrict__ nbr8, size_t stride, uint32_t i, uint32_t nF, int l,
+                                       Load&& load, Body&& body) {
+  if constexpr (L == 1) {
+    for_fluid_groups<G>(nbr8, stride, i, nF, load, body);
+  } else {
+    static_assert(L == 4, "a pack holds four pairs of slots");
+    const uint32_t* __restrict__ words = reinterpret_cast<const uint32_t*>(nbr8);
+    const uint32_t np = (nF + PACK - 1) / PACK;
+    const uint32_t last = np > 0 ? np - 1 : 0;
+    auto word = [&](uint32_t p) { return words[((size_t)min(p, last) * stride + i) * 4 + l]; };
+    uint32_t a = word(0), b = word(1), a2 = word(2), b2 = word(3);
+#pragma unroll 1
+    for (uint32_t p = 0; p < np; p += 2) {
+      const uint32_t s0 = a & 0xffffu, s1 = a >> 16, s2 = b & 0xffffu, s3 = b >> 16;
+      a = a2; b = b2;
+      a2 = word(p + 4); b2 = word(p + 5);
+      const uint32_t e = p * PACK + 2u * (uint32_t)l;
+      // rows past the last one repeat it: their slots are not live
+      const auto v0 = load(s0), v1 = load(s1), v2 = load(s2), v3 = load(s3);
+      body(v0, e < nF);
+      body(v1, e + 1u < nF);
+      body(v2, e + (uint32_t)PACK < nF);
+      body(v3, e + (uint32_t)PACK + 1u < nF);
+    }
+  }
+}
+
+// Sum over the L lanes of a particle (consecutive lanes), in every lane.
+template <int L> __device__ inline float lane_sum(float x) {
+  if constexpr (L == 4) {
+    x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
+    x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
+  }
+  return x;
+}
+
 // Visits the nB boundary neighbours of particle i in list order, G at a time:
 // the group's sample indices are loaded first, then the group's sample data
 // (`load(j)`), so a group costs two dependent trips to memory instead of two
-// per neighbour; `body(v, j)` then runs for the group's neighbours in order.
-template <uint32_t G = 4, class Load, class Body>
+// per neighbour; `body(v, j, u)` then runs for the group's neighbours in order,
+// u their place in the group.
+// With L lanes per particle, lane l takes every L-th neighbour from l on.
+template <uint32_t G = 4, uint32_t L = 1, class Load, class Body>
 __device__ inline void for_boundary_groups(const uint32_t* __restrict__ nbrB, size_t stride, uint32_t i,
-                                           uint32_t nB, Load&& load, Body&& body) {
+                                           uint32_t nB, Load&& load, Body&& body, uint32_t l = 0) {
 #pragma unroll 1
-  for (uint32_t k0 = 0; k0 < nB; k0 += G) {
+  for (uint32_t k0 = l; k0 < nB; k0 += G * L) {
     uint32_t jj[G];
 #pragma unroll
-    for (uint32_t u = 0; u < G; ++u) jj[u] = nbrB[(size_t)min(k0 + u, nB - 1) * stride + i];
+    for (uint32_t u = 0; u < G; ++u) jj[u] = nbrB[(size_t)min(k0 + u * L, nB - 1) * stride + i];
     decltype(load(0u)) v[G];
 #pragma unroll
     for (uint32_t u = 0; u < G; ++u) v[u] = load(jj[u]);
 #pragma unroll
     for (uint32_t u = 0; u < G; ++u)
-      if (k0 + u < nB) body(v[u], jj[u]);
+      if (k0 + u * L < nB) body(v[u], jj[u], u);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Four lanes per particle in the step's own passes (L = 4: small scenes, see
+// gather_parts_log2).  The lanes of a quad evaluate different pairs; every lane
+// then adds all pairs' terms in list order, reading each from the lane that has
+// it (a quad broadcast costs one instruction), so the sums are those of one lane
+// per particle bit for bit.  `term` forms what a pair contributes (Terms), `acc`
+// adds it; with L = 1 they run one after the other.  This pays for two to four
+// terms a pair: the reverse passes' seven to twelve took 9.2 us in place of 6.7
+// (delta, 2,000 particles).
+// ---------------------------------------------------------------------------
+template <int N> struct Terms {
+  float f[N];
+};
+template <int K, int N> __device__ inline Terms<N> quad_bcast(const Terms<N>& t) {
+  Terms<N> o;
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+    o.f[n] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t.f[n]), K * 0x55, 0xf, 0xf, true));
+  return o;
+}
+
+// Fluid pairs: lane l of the quad takes slots 2 l and 2 l + 1 of each pack.
+template <int G, int L, class Load, class Term, class Acc>
+__device__ inline void for_fluid_terms(const uint4* __restrict__ nbr8, size_t stride, uint32_t i, uint32_t nF, int l,
+                                       Load&& load, Term&& term, Acc&& acc) {
+  if constexpr (L == 1) {
+    for_fluid_groups<G>(nbr8, stride, i, nF, load, [&](const auto& v, bool live) { acc(term(v, live)); });
+  } else {
+    static_assert(L == 4, "a pack holds four pairs of slots");
+    const uint32_t* __restrict__ words = reinterpret_cast<const uint32_t*>(nbr8);
+    const uint32_t np = (nF + PACK - 1) / PACK;
+    const uint32_t last = np > 0 ? np - 1 : 0;
+    auto word = [&](uint32_t p) { return words[((size_t)min(p, last) * stride + i) * 4 + l]; };
+    uint32_t w0 = word(0), w1 = word(1), w2 = word(2);
+#pragma unroll 1
+    for (uint32_t p = 0; p < np; ++p) {
+      const uint32_t s0 = w0 & 0xffffu, s1 = w0 >> 16;
+      w0 = w1; w1 = w2; w2 = word(p + 3);
+      const uint32_t e = p * PACK + 2u * (uint32_t)l;
+      const auto v0 = load(s0), v1 = load(s1);
+      const auto t0 = term(v0, e < nF), t1 = term(v1, e + 1u < nF);
+      acc(quad_bcast<0>(t0)); acc(quad_bcast<0>(t1));
+      acc(quad_bcast<1>(t0)); acc(quad_bcast<1>(t1));
+      acc(quad_bcast<2>(t0)); acc(quad_bcast<2>(t1));
+      acc(quad_bcast<3>(t0)); acc(quad_bcast<3>(t1));
+    }
+  }
+}
+
+// Which product of a boundary pair's three is rounded by itself, and whether its
+// share is added fused, has always gone by the neighbour's place u in its group
+// of the one-lane loop; both forms take it from u, so that a particle's sums are
+// the same bits by either.
+__device__ inline float place_dot(uint32_t u, float ax, float ay, float az, float bx, float by, float bz) {
+  const bool x_first = (u & 2u) == 0u;
+  const float a0 = x_first ? ax : ay, b0 = x_first ? bx : by, a1 = x_first ? ay : ax, b1 = x_first ? by : bx;
+  return fmaf(az, bz, fmaf(a1, b1, a0 * b0));
+}
+
+// Boundary samples: lane l of the quad takes neighbours l and l + 4 of each
+// eight; `term(v, j, u)` runs once per neighbour (its side effects too), u the
+// neighbour's place in its group of G.
+template <uint32_t G, int L, class Load, class Term, class Acc>
+__device__ inline void for_boundary_terms(const uint32_t* __restrict__ nbrB, size_t stride, uint32_t i, uint32_t nB,
+                                          int l, Load&& load, Term&& term, Acc&& acc) {
+  static_assert(4 % G == 0, "a lane's neighbours have one place in their groups");
+  if constexpr (L == 1) {
+    for_boundary_groups<G>(nbrB, stride, i, nB, load,
+                           [&](const auto& v, uint32_t j, uint32_t u) { acc(term(v, j, u), u); });
+  } else {
+#pragma unroll 1
+    for (uint32_t k0 = 0; k0 < nB; k0 += 8) {
+      const uint32_t ka = k0 + (uint32_t)l, kb = ka + 4u, u = (uint32_t)l % G;
+      const uint32_t ja = nbrB[(size_t)min(ka, nB - 1) * stride + i], jb = nbrB[(size_t)min(kb, nB - 1) * stride + i];
+      const auto va = load(ja), vb = load(jb);
+      decltype(term(va, ja, u)) ta{}, tb{};
+      if (ka < nB) ta = term(va, ja, u);
+      if (kb < nB) tb = term(vb, jb, u);
+      acc(quad_bcast<0>(ta), 0u);
+      if (k0 + 1 < nB) acc(quad_bcast<1>(ta), 1u % G);
+      if (k0 + 2 < nB) acc(quad_bcast<2>(ta), 2u % G);
+      if (k0 + 3 < nB) acc(quad_bcast<3>(ta), 3u % G);
+      if (k0 + 4 < nB) acc(quad_bcast<0>(tb), 0u);
+      if (k0 + 5 < nB) acc(quad_bcast<1>(tb), 1u % G);
+      if (k0 + 6 < nB) acc(quad_bcast<2>(tb), 2u % G);
+      if (k0 + 7 < nB) acc(quad_bcast<3>(tb), 3u % G);
+    }
   }
 }
 
@@ -243,11 +391,16 @@ struct Slot8 {
 
 // Same visit order without unrolling, for the global-memory fallback (a halo
 // beyond the LDS capacity): keeps the rare path out of the unrolled hot loop.
-template <class Body>
+// With four lanes per particle, lane l takes the slots it takes from LDS.
+template <int L = 1, class Body>
 __device__ inline void for_fluid_slots_rolled(const uint4* __restrict__ nbr8, size_t stride, uint32_t i,
-                                              uint32_t nF, Body&& body) {
+                                              uint32_t nF, Body&& body, int l = 0) {
+  constexpr uint32_t W = PACK / L;  // slots of a pack that a lane takes
 #pragma unroll 1
-  for (uint32_t k = 0; k < nF; ++k) {
+  for (uint32_t m = 0;; ++m) {
+    const uint32_t k = (m / W) * PACK + W * (uint32_t)l + m % W;
+    if ((m / W) * PACK >= nF) break;
+    if (k >= nF) continue;
     const uint4 v = nbr8[(size_t)(k >> 3) * stride + i];
     body(pack_get(v, (int)(k & 7u)));
   }

@@ -234,6 +234,243 @@ k_build_tiled(const float4* __restrict__ pos, int nf, GridDesc g, const uint32_t
 }
 
 // ---------------------------------------------------------------------------
+// The same lists for scenes of a few bricks, where the build costs one
+// wavefront's chain.  A wavefront takes up to eight particles of one cell: the
+// particles share their candidates (nine rows of three halo cells, about 270 at
+// rest density), so the lanes hold the candidates, 64 a round, and the
+// particles are tested one after the other against a whole round; the accept
+// mask is a ballot, a slot's place in the list its rank in the mask, and the
+// particle itself drops out by its slot.  2^cell_parts_log2 workgroups share a
+// brick, each with the whole halo and its share of the 64 cells.
+// Against k_build_tiled, us: 1,000 particles 15 (45), 8,000 22 (44), 28,000 35
+// (48), 56,000 53 (61); from 98,000 (79 against 72) the scalar work per round
+// costs more than the short chains give.
+// ---------------------------------------------------------------------------
+constexpr int CNR = 6;             // rounds of 64 candidates kept in registers
+constexpr int CP = 8;              // particles a wavefront takes at a time
+constexpr int BW = BB / 64;
+__device__ inline uint32_t rfl(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ inline uint32_t rdl(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
+__device__ inline float rdl(float v, int lane) { return __uint_as_float(rdl(__float_as_uint(v), lane)); }
+// rank of this lane among the set bits of a wave mask, plus base
+__device__ inline uint32_t mask_rank(unsigned long long m, uint32_t base) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
+}
+
+__global__ void __launch_bounds__(BB)
+k_build_cells(const float4* __restrict__ pos, int nf, GridDesc g, const uint32_t* __restrict__ fstart,
+              const float4* __restrict__ bpos, const uint32_t* __restrict__ bstart,
+              const uint32_t* __restrict__ bperm, float h2, int maxb, int cap, int cell_parts_log2,
+              uint4* __restrict__ nbr8, uint32_t* __restrict__ nbrB, uint32_t* __restrict__ cnt,
+              uint32_t* __restrict__ overflow, uint4* __restrict__ thdr, uint32_t* __restrict__ tmap) {
+  __shared__ TileHdr<BB> T;
+  __shared__ uint32_t bcs[HALO], bcn[HALO];  // boundary sample range of each halo cell
+  __shared__ uint32_t bpre[BW][28];          // boundary candidates before each of a cell's 27 neighbour cells
+  __shared__ __attribute__((aligned(16))) uint16_t list[BW][CP][MAXF];
+  __shared__ uint32_t next_item;
+  extern __shared__ float lds[];
+  const uint32_t blk = xcd_block();
+  const uint32_t brick = blk >> cell_parts_log2, part = blk & ((1u << cell_parts_log2) - 1u);
+  if (brick_empty(fstart, brick)) {
+    if (threadIdx.x == 0 && part == 0u) thdr[brick] = make_uint4(0u, 0u, 0u, 0u);
+    return;
+  }
+  tile_setup<BB>(g, fstart, brick, T);
+  if (threadIdx.x == 0 && part == 0u) thdr[brick] = make_uint4(T.own_begin, T.own_end, T.total, 0u);
+  const uint32_t total = T.total;
+  const int t = threadIdx.x;
+  if (t == 0 && part == 0u) atomicMax(&overflow[3], total);
+  if (total > 65535u) {
+    // tile slots are 16-bit: leave empty lists (safe for every pass) and report
+    if (part == 0u)
+      for (uint32_t i = T.own_begin + t; i < T.own_end; i += BB) cnt[i] = 0u;
+    if (t == 0) atomicMax(&overflow[0], total);
+    return;
+  }
+  if (t < HALO) {
+    const int cx = 4 * T.bx - 1 + t % 6, cy = 4 * T.by - 1 + (t / 6) % 6, cz = 4 * T.bz - 1 + t / 36;
+    uint32_t st = 0, n = 0;
+    if (cx >= 0 && cy >= 0 && cz >= 0 && cx < g.n[0] && cy < g.n[1] && cz < g.n[2]) {
+      const uint32_t key = cell_key(g, cx, cy, cz);
+      st = bstart[key];
+      n = bstart[key + 1] - st;
+    }
+    bcs[t] = st;
+    bcn[t] = n;
+  }
+  // items: four per cell, item m of a cell takes its particles 8 m.. + 8 (and every 32nd from there)
+  const uint32_t item_end = (part + 1u) * (256u >> cell_parts_log2);
+  if (t == 0) next_item = part * (256u >> cell_parts_log2);
+  const bool in_lds = total <= (uint32_t)min(cap, BSTRIDE - 4);
+  float* lx = lds; float* ly = lds + BSTRIDE; float* lz = lds + 2 * BSTRIDE;
+  constexpr int PTB = per_thread<BB>();
+  uint32_t js[PTB];
+  tile_indices<BB>(T, min(total, (uint32_t)TILE_CAP), js);
+#pragma unroll
+  for (int r = 0; r < PTB; ++r) {
+    const uint32_t s = t + r * BB;
+    if (part == 0u && s < min(total, (uint32_t)TILE_CAP)) tmap[(size_t)brick * TILE_CAP + s] = js[r];
+  }
+  if (in_lds) {
+    float4 q[PTB];
+#pragma unroll
+    for (int r = 0; r < PTB; ++r)
+      if (t + r * BB < (int)total) q[r] = pos[js[r]];
+#pragma unroll
+    for (int r = 0; r < PTB; ++r) {
+      const uint32_t s = t + r * BB;
+      if (s < total) { lx[s] = q[r].x; ly[s] = q[r].y; lz[s] = q[r].z; }
+    }
+  }
+  __syncthreads();
+  const size_t stride = (size_t)nf;
+  const int lane = t & 63;
+  const int wv = (int)rfl((uint32_t)t >> 6);
+  while (true) {
+    uint32_t item = 0;
+    if (lane == 0) item = atomicAdd(&next_item, 1u);
+    item = rfl(item);
+    if (item >= item_end) break;
+    const uint32_t cell = item >> 2;
+    // cell coordinates in the brick from its Morton number
+    const int x = (int)((cell & 1u) | ((cell >> 2) & 2u)), y = (int)(((cell >> 1) & 1u) | ((cell >> 3) & 2u)),
+              z = (int)(((cell >> 2) & 1u) | ((cell >> 4) & 2u));
+    const int hc0 = (z + 1) * 36 + (y + 1) * 6 + (x + 1);
+    const uint32_t self0 = rfl(T.coff[hc0]);
+    const uint32_t own = rfl(T.coff[hc0 + 1]) - self0;
+    if ((item & 3u) * CP >= own) continue;
+    const uint32_t i0 = rfl(T.cstart[hc0]);
+    // candidate t of row r is slot t + off[r]; the row starts at candidate pre[r]
+    uint32_t off[9], pre[9], ncand = 0;
+    {
+      const int rr = min(lane, 8);
+      const int hm = hc0 + (rr / 3 - 1) * 36 + (rr % 3 - 1) * 6 - 1;
+      const uint32_t v0 = T.coff[hm], v1 = T.coff[hm + 3];
+#pragma unroll
+      for (int r = 0; r < 9; ++r) {
+        const uint32_t r0 = rdl(v0, r);
+        pre[r] = ncand;
+        off[r] = r0 - ncand;
+        ncand += rdl(v1, r) - r0;
+      }
+    }
+    // boundary candidates of the 27 cells
+    uint32_t nbc = 0;
+    {
+      uint32_t n = 0;
+      if (lane < 27) n = bcn[hc0 + (lane / 9 - 1) * 36 + ((lane / 3) % 3 - 1) * 6 + (lane % 3 - 1)];
+      if (__ballot(n > 0u) != 0ull) {
+        uint32_t inc = n;
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+          const uint32_t u = __shfl_up(inc, o, 64);
+          if (lane >= o) inc += u;
+        }
+        if (lane < 27) bpre[wv][lane] = inc - n;
+        nbc = rdl(inc, 26);
+        __threadfence_block();
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    float qx[CNR], qy[CNR], qz[CNR];
+    uint32_t sl[CNR];
+    bool loaded = false;
+    for (uint32_t b0 = (item & 3u) * CP; b0 < own; b0 += 4 * CP) {
+      const uint32_t nk = min(own - b0, (uint32_t)CP);
+      // lanes 0..7 hold the particles
+      float px = 0.f, py = 0.f, pz = 0.f;
+      if ((uint32_t)lane < nk) {
+        const float4 p = pos[i0 + b0 + lane];
+        px = p.x; py = p.y; pz = p.z;
+      }
+      uint32_t myF = 0, myB = 0;  // counts of particle b0 + lane / 8
+      for (uint32_t g0 = 0; g0 < ncand; g0 += CNR * 64) {
+        if (!loaded) {
+#pragma unroll
+          for (int r = 0; r < CNR; ++r) {
+            const uint32_t tc = g0 + r * 64 + lane;
+            uint32_t o = off[0];
+#pragma unroll
+            for (int w = 1; w < 9; ++w) o = tc >= pre[w] ? off[w] : o;
+            const uint32_t s = tc + o;
+            sl[r] = s;
+            qx[r] = 1.0e30f; qy[r] = 0.f; qz[r] = 0.f;  // no candidate: never within reach
+            if (tc < ncand) {
+              if (in_lds) {
+                qx[r] = lx[s]; qy[r] = ly[s]; qz[r] = lz[s];
+              } else {
+                const float4 q = pos[tile_global<BB>(T, s)];
+                qx[r] = q.x; qy[r] = q.y; qz[r] = q.z;
+              }
+            }
+          }
+          loaded = ncand <= (uint32_t)(CNR * 64);
+        }
+        for (uint32_t k = 0; k < nk; ++k) {
+          const uint32_t ps = self0 + b0 + k;
+          const float kx = rdl(px, (int)k), ky = rdl(py, (int)k), kz = rdl(pz, (int)k);
+          uint16_t* L = list[wv][k];
+          uint32_t n = g0 == 0u ? 0u : rdl(myF, (int)(8u * k));
+#pragma unroll
+          for (int r = 0; r < CNR; ++r) {
+            if (g0 + r * 64u >= ncand) break;
+            const bool hit = dist2_exact(kx, ky, kz, qx[r], qy[r], qz[r]) < h2 && sl[r] != ps;
+            const unsigned long long m = __ballot(hit);
+            const uint32_t at = mask_rank(m, n);
+            if (hit && at < (uint32_t)MAXF) L[at] = (uint16_t)sl[r];
+            n += (uint32_t)__popcll(m);
+          }
+          if ((uint32_t)(lane >> 3) == k) myF = n;
+        }
+      }
+      for (uint32_t g0 = 0; g0 < nbc; g0 += 64) {
+        const uint32_t tc = g0 + lane;
+        uint32_t j = 0;
+        float bx = 1.0e30f, by = 0.f, bz = 0.f;
+        if (tc < nbc) {
+          int lo = 0, hi = 26;  // the cell holding candidate tc
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (bpre[wv][mid] <= tc) lo = mid; else hi = mid - 1;
+          }
+          j = bperm[bcs[hc0 + (lo / 9 - 1) * 36 + ((lo / 3) % 3 - 1) * 6 + (lo % 3 - 1)] + (tc - bpre[wv][lo])];
+          const float4 q = bpos[j];
+          bx = q.x; by = q.y; bz = q.z;
+        }
+        for (uint32_t k = 0; k < nk; ++k) {
+          const bool hit = dist2_exact(rdl(px, (int)k), rdl(py, (int)k), rdl(pz, (int)k), bx, by, bz) < h2;
+          const unsigned long long m = __ballot(hit);
+          const uint32_t at = mask_rank(m, rdl(myB, (int)(8u * k)));
+          if (hit && at < (uint32_t)maxb) nbrB[(size_t)at * stride + (i0 + b0 + k)] = j;
+          if ((uint32_t)(lane >> 3) == k) myB += (uint32_t)__popcll(m);
+        }
+      }
+      // the lists leave: eight lanes per particle, a 16-byte pack each
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
+      const uint32_t k = (uint32_t)lane >> 3;
+      if (k < nk) {
+        const uint32_t i = i0 + b0 + k;
+        const uint32_t nF = min(myF, (uint32_t)MAXF), nB = min(myB, (uint32_t)maxb);
+        for (uint32_t p = lane & 7u; p * PACK < nF; p += 8) {
+          uint4 v = *reinterpret_cast<const uint4*>(&list[wv][k][p * PACK]);
+          const uint32_t left = nF - p * PACK;  // entries past the list's end are slot 0
+          auto keep = [&](uint32_t w, uint32_t e) { return left >= e + 2u ? w : (left > e ? w & 0xffffu : 0u); };
+          nbr8[(size_t)p * stride + i] = make_uint4(keep(v.x, 0), keep(v.y, 2), keep(v.z, 4), keep(v.w, 6));
+        }
+        if ((lane & 7) == 0) {
+          if (myF > (uint32_t)MAXF) atomicMax(&overflow[0], myF);
+          if (myB > (uint32_t)maxb) atomicMax(&overflow[2], myB);
+          cnt[i] = nF | (nB << 16);
+        }
+      }
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Gather passes: PASS_BLOCK threads per brick.  Dynamic LDS per slot:
 // x, y, z (+ per-pass fields).
 // ---------------------------------------------------------------------------
@@ -241,8 +478,8 @@ constexpr int PB = PASS_BLOCK;
 constexpr int PT = per_thread<PB>();
 // The velocity update stages 4 floats per slot, so LDS would fit four 640-thread
 // workgroups but the CU holds at most 32 wavefronts: 512 threads keep four.
-constexpr int VB = 512;
-constexpr int VT = per_thread<VB>();
+// With four lanes per particle a workgroup's 160 particles fill 640 threads.
+template <int L> constexpr int velocity_block() { return L == 1 ? 512 : PASS_BLOCK; }
 
 // TimeStep::computeDensities (TimeStep.cpp:147-202) + computeDFSPHFactor
 // (TimeStepDiffDFSPH.cpp:883-962) + the first loop of warmstartDivergenceSolve
@@ -254,10 +491,9 @@ k_density_factor_t(PassArgs a, float* __restrict__ rho, float* __restrict__ alph
   __shared__ TileHdr<PB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   BrickView B;
-  if (!brick_open<PB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<PB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
   float4* LA = lds4;                                          // x, y, z, vx
@@ -265,7 +501,7 @@ k_density_factor_t(PassArgs a, float* __restrict__ rho, float* __restrict__ alph
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[PT];
-    map_indices<PB>(a.tmap, brick, total, js);
+    map_indices<PB>(a.tmap, B.brick, total, js);
     float4 q[PT], v[PT];
 #pragma unroll
     for (int r = 0; r < PT; ++r)
@@ -326,7 +562,7 @@ k_density_factor_t(PassArgs a, float* __restrict__ rho, float* __restrict__ alph
     for_boundary_groups(
         a.nbrB, stride, i, nB,
         [&](uint32_t j) { return Slot8{a.bpos[j], divergence_on ? a.bvel[j] : make_float4(0.f, 0.f, 0.f, 0.f)}; },
-        [&](const Slot8& s, uint32_t) {
+        [&](const Slot8& s, uint32_t, uint32_t) {
           const float4 q = s.a, vb = s.b;
           const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
           const PairKernel kw = cubic_pair(c.K, rx * rx + ry * ry + rz * rz);
@@ -360,24 +596,24 @@ k_density_factor_t(PassArgs a, float* __restrict__ rho, float* __restrict__ alph
 // -dt k_i grad_p_ib and receives f = -m_i dv / dt (BoundaryModel::addForce,
 // BoundaryModel.h:46-58), summed here in FP64 per dynamic body.
 // LDS per slot: x, y, z, k.
+template <int L, int VB>
 __global__ void __launch_bounds__(VB) __attribute__((amdgpu_waves_per_eu(8, 8)))
 k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restrict__ kappa_acc,
                     RigidDev* __restrict__ rig, const int* __restrict__ stop, IterTapeOut tape) {
+  constexpr int VT = per_thread<VB>();
   __shared__ TileHdr<VB> T;
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
   if (stop && *stop) return;
-  const uint32_t brick = xcd_block();
-  const int cap = a.cap;
   BrickView B;
-  if (!brick_open<VB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) return;
+  if (!brick_open<VB>(a, T, B)) return;
   const uint32_t total = B.total;
   const bool in_lds = B.in_lds;
-  float4* L = lds4;  // x, y, z, k
+  float4* LS = lds4;  // x, y, z, k
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[VT];
-    map_indices<VB>(a.tmap, brick, total, js);
+    map_indices<VB>(a.tmap, B.brick, total, js);
     float4 q[VT];
     float kk[VT];
 #pragma unroll
@@ -386,7 +622,7 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
 #pragma unroll
     for (int r = 0; r < VT; ++r) {
       const uint32_t s = t + r * VB;
-      if (s < total) L[s] = make_float4(q[r].x, q[r].y, q[r].z, kk[r]);
+      if (s < total) LS[s] = make_float4(q[r].x, q[r].y, q[r].z, kk[r]);
     }
   }
   __syncthreads();
@@ -395,18 +631,21 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
   // The particle loop runs the same number of times on every lane of a wave, so
   // the coupling partials of each round are reduced over the wave at its end
   // (and are not live across the next round's fluid pair loop).
-  for (uint32_t base = B.own_begin; base < B.own_end; base += VB) {
-    const uint32_t i = base + t;
+  const int l = t % L;  // lane of the particle
+  for (uint32_t base = B.own_begin; base < B.own_end; base += VB / L) {
+    const uint32_t i = base + t / L;
     int cb = -1;
     double F0 = 0, F1 = 0, F2 = 0, T0 = 0, T1 = 0, T2 = 0;
     if (i < B.own_end) {
       const float ki = kfield[i];
-      if (kappa_acc) kappa_acc[i] += ki;
       const float4 p = a.pos[i];
       float4 vi = a.vel[i];
-      if (tape.v) tape.v[i] = vi;
-      if (tape.k) tape.k[i] = ki;
-      if (tape.b) tape.b[i] = tape.bsrc[i];
+      if (l == 0) {
+        if (kappa_acc) kappa_acc[i] += ki;
+        if (tape.v) tape.v[i] = vi;
+        if (tape.k) tape.k[i] = ki;
+        if (tape.b) tape.b[i] = tape.bsrc[i];
+      }
       const uint32_t cc = a.cnt[i];
       const uint32_t nF = cc & 0xffffu, nB = cc >> 16;
       // v_i -= dt (k_i + k_j) grad_p_ij = dt V_f (k_i + k_j) c_ij r_ij; dt V_f applied once
@@ -416,16 +655,19 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
         const float kSum = ki + kj;
         const float rx = p.x - qx, ry = p.y - qy, rz = p.z - qz;
         const float s = kSum * cubic_grad_c(c.K, rx * rx + ry * ry + rz * rz, live && fabsf(kSum) > c.eps);
-        ux += s * rx; uy += s * ry; uz += s * rz;
+        return Terms<4>{{s, rx, ry, rz}};
+      };
+      auto add = [&](const Terms<4>& q) {
+        ux += q.f[0] * q.f[1]; uy += q.f[0] * q.f[2]; uz += q.f[0] * q.f[3];
       };
       if (in_lds) {
-        for_fluid_groups<2>(a.nbr8, stride, i, nF, [&](uint32_t s) { return L[s]; },
-                            [&](const float4& q, bool live) { pair(q.x, q.y, q.z, q.w, live); });
+        for_fluid_terms<2, L>(a.nbr8, stride, i, nF, l, [&](uint32_t s) { return LS[s]; },
+                              [&](const float4& q, bool live) { return pair(q.x, q.y, q.z, q.w, live); }, add);
       } else {
         for_fluid_slots_rolled(a.nbr8, stride, i, nF, [&](uint32_t s) {
           const uint32_t j = tile_global<VB>(T, s);
           const float4 q = a.pos[j];
-          pair(q.x, q.y, q.z, kfield[j], true);
+          add(pair(q.x, q.y, q.z, kfield[j], true));
         });
       }
       {
@@ -434,13 +676,12 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
       }
       if (fabsf(ki) > c.eps) {
         auto load = [&](uint32_t j) { return a.bpos[j]; };
-        for_boundary_groups<2>(a.nbrB, stride, i, nB, load, [&](const float4& q, uint32_t j) {
+        for_boundary_terms<2, L>(a.nbrB, stride, i, nB, l, load, [&](const float4& q, uint32_t j, uint32_t) {
           const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
           const float sc = cubic_grad_c(c.K, rx * rx + ry * ry + rz * rz);
           const float gpx = -q.w * (sc * rx), gpy = -q.w * (sc * ry), gpz = -q.w * (sc * rz);
           const float am = -c.dt * 1.f * ki;
           const float dvx = am * gpx, dvy = am * gpy, dvz = am * gpz;
-          vi.x += dvx; vi.y += dvy; vi.z += dvz;
           if ((int)j >= a.nb_static) {
             const int body = (int)a.bx0[j].w;
             if (rig[body].dynamic) {
@@ -457,9 +698,19 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
               T0 += ryd * fz - rzd * fy; T1 += rzd * fx - rxd * fz; T2 += rxd * fy - ryd * fx;
             }
           }
+          return Terms<3>{{gpx, gpy, gpz}};
+        }, [&](const Terms<3>& q, uint32_t u) {
+          const float am = -c.dt * 1.f * ki;
+          if (u == 0u) {
+#pragma clang fp contract(off)
+            const float dx = am * q.f[0], dy = am * q.f[1], dz = am * q.f[2];
+            vi.x += dx; vi.y += dy; vi.z += dz;
+          } else {
+            vi.x = fmaf(am, q.f[0], vi.x); vi.y = fmaf(am, q.f[1], vi.y); vi.z = fmaf(am, q.f[2], vi.z);
+          }
         });
       }
-      a.vel[i] = vi;
+      if (l == 0) a.vel[i] = vi;
     }
     // Wave-level FP64 reduction of the round's coupling partials, one body at a time.
     while (true) {
@@ -487,6 +738,7 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
 // and k_i = b_i alpha_i kcoef for the next Jacobi update (mode 0 divergence,
 // 1 pressure); mode 2 is the first loop of warmstartPressureSolve (:987-999).
 // LDS per slot: x, y, z, vx, vy, vz.
+template <int L>
 __global__ void __launch_bounds__(PB) __attribute__((amdgpu_waves_per_eu(6, 8)))
 k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, const float* __restrict__ alpha,
               float* __restrict__ badv, float* __restrict__ kf, float* __restrict__ kappa, double* __restrict__ err,
@@ -495,12 +747,11 @@ k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, 
   extern __shared__ float4 lds4[];
   const StepConst& c = a.c;
   if (stop && *stop) return;
-  const uint32_t brick = xcd_block();
   const int cap = a.cap;
   const bool residual = err && (mode == RECOMPUTE_DIV || mode == RECOMPUTE_PRESSURE);
   BrickView B;
-  if (!brick_open<PB>(a.g, a.fstart, a.thdr, brick, cap, T, B)) {
-    if (residual && threadIdx.x == 0) err[brick] = 0.0;
+  if (!brick_open<PB>(a, T, B)) {
+    if (residual && threadIdx.x == 0) err[B.block] = 0.0;
     return;
   }
   const uint32_t total = B.total;
@@ -510,7 +761,7 @@ k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, 
   const int t = threadIdx.x;
   if (in_lds) {
     uint32_t js[PT];
-    map_indices<PB>(a.tmap, brick, total, js);
+    map_indices<PB>(a.tmap, B.brick, total, js);
     float4 q[PT], v[PT];
 #pragma unroll
     for (int r = 0; r < PT; ++r)
@@ -527,7 +778,8 @@ k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, 
   __syncthreads();
   const size_t stride = (size_t)c.nf;
   double e = 0.0;
-  for (uint32_t i = B.own_begin + t; i < B.own_end; i += PB) {
+  const int l = t % L;  // lane of the particle
+  for (uint32_t i = B.own_begin + t / L; i < B.own_end; i += PB / L) {
     const float4 p = a.pos[i];
     const float4 vi = a.vel[i];
     const uint32_t cc = a.cnt[i];
@@ -537,29 +789,32 @@ k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, 
     auto pair = [&](float qx, float qy, float qz, float vx, float vy, float vz, bool live) {
       const float rx = p.x - qx, ry = p.y - qy, rz = p.z - qz;
       const float sc = cubic_grad_c(c.K, rx * rx + ry * ry + rz * rz, live);
-      fdelta += sc * ((vi.x - vx) * rx + (vi.y - vy) * ry + (vi.z - vz) * rz);
+      return Terms<2>{{sc, (vi.x - vx) * rx + (vi.y - vy) * ry + (vi.z - vz) * rz}};
     };
+    auto add = [&](const Terms<2>& q) { fdelta += q.f[0] * q.f[1]; };
     if (in_lds) {
-      for_fluid_groups<4>(a.nbr8, stride, i, nF, [&](uint32_t s) { return Slot6{LA[s], LB[s]}; },
-                          [&](const Slot6& q, bool live) {
-                            pair(q.a.x, q.a.y, q.a.z, q.a.w, q.b.x, q.b.y, live);
-                          });
+      for_fluid_terms<4, L>(a.nbr8, stride, i, nF, l, [&](uint32_t s) { return Slot6{LA[s], LB[s]}; },
+                            [&](const Slot6& q, bool live) {
+                              return pair(q.a.x, q.a.y, q.a.z, q.a.w, q.b.x, q.b.y, live);
+                            }, add);
     } else {
       for_fluid_slots_rolled(a.nbr8, stride, i, nF, [&](uint32_t s) {
         const uint32_t j = tile_global<PB>(T, s);
         const float4 q = a.pos[j];
         const float4 v = a.vel[j];
-        pair(q.x, q.y, q.z, v.x, v.y, v.z, true);
+        add(pair(q.x, q.y, q.z, v.x, v.y, v.z, true));
       });
     }
     delta = c.V_f * fdelta;
-    for_boundary_groups(a.nbrB, stride, i, nB, [&](uint32_t j) { return Slot8{a.bpos[j], a.bvel[j]}; },
-                        [&](const Slot8& s, uint32_t) {
-                          const float4 q = s.a, vb = s.b;
-                          const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
-                          const float sc = cubic_grad_c(c.K, rx * rx + ry * ry + rz * rz);
-                          delta += q.w * sc * ((vi.x - vb.x) * rx + (vi.y - vb.y) * ry + (vi.z - vb.z) * rz);
-                        });
+    for_boundary_terms<4, L>(a.nbrB, stride, i, nB, l, [&](uint32_t j) { return Slot8{a.bpos[j], a.bvel[j]}; },
+                             [&](const Slot8& s, uint32_t, uint32_t u) {
+                               const float4 q = s.a, vb = s.b;
+                               const float rx = p.x - q.x, ry = p.y - q.y, rz = p.z - q.z;
+                               const float sc = cubic_grad_c(c.K, place_dot(u, rx, ry, rz, rx, ry, rz));
+                               return Terms<2>{{q.w * sc, place_dot(u, vi.x - vb.x, vi.y - vb.y, vi.z - vb.z,
+                                                                       rx, ry, rz)}};
+                             }, [&](const Terms<2>& q, uint32_t) { delta += q.f[0] * q.f[1]; });
+    if (l != 0) continue;
     float b;
     if (mode == 0) {
       b = fmaxf(delta, 0.f);
@@ -581,7 +836,7 @@ k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, 
     }
     badv[i] = b;
   }
-  if (residual) block_sum_double<PB>(e, err + brick);
+  if (residual) block_sum_double<PB>(e, err + B.block);
 }
 
 // Expands tile slots back to sorted fluid indices (diagnostics).
@@ -602,34 +857,51 @@ k_expand_lists(GridDesc g, const uint32_t* __restrict__ fstart, int nf, const ui
 
 // ---------------------------------------------------------------------------
 
+int gather_parts_log2(int nf) {
+  return nf < 40000 ? 2 : nf < 80000 ? 1 : 0;
+}
+
 void launch_build_tiled(FluidBufs& f, BoundaryBufs& b, const GridDesc& g, GridBufs& gb, NbrBufs& nb, float h2,
                         hipStream_t s) {
   const size_t shm = sizeof(float) * 3 * (size_t)BSTRIDE;
-  hipLaunchKernelGGL(k_build_tiled, dim3(nbricks(g)), dim3(BB), shm, s, f.pos, f.n, g, gb.fstart, b.pos, gb.bstart,
-                     gb.bperm, h2, nb.maxb, nb.cap, nb.nbr8, nb.nbrB, nb.cnt, nb.overflow, nb.thdr, nb.tmap);
+  // workgroups per brick of k_build_cells: 2,000 particles 17 us with 8, 21 with 4; 28,000: 41 and 35
+  const int cell_parts_log2 = f.n < 16384 ? 3 : 2;
+  if (nb.parts_log2 > 0)
+    hipLaunchKernelGGL(k_build_cells, dim3(nbricks(g) << cell_parts_log2), dim3(BB), shm, s, f.pos, f.n, g, gb.fstart,
+                       b.pos, gb.bstart, gb.bperm, h2, nb.maxb, nb.cap, cell_parts_log2, nb.nbr8, nb.nbrB, nb.cnt,
+                       nb.overflow, nb.thdr, nb.tmap);
+  else
+    hipLaunchKernelGGL(k_build_tiled, dim3(nbricks(g)), dim3(BB), shm, s, f.pos, f.n, g, gb.fstart, b.pos, gb.bstart,
+                       gb.bperm, h2, nb.maxb, nb.cap, nb.nbr8, nb.nbrB, nb.cnt, nb.overflow, nb.thdr, nb.tmap);
 }
 
 void launch_density_factor_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidBufs& f, BoundaryBufs& b,
                              NbrBufs& nb, int div_warm, int divergence_on, float2* aux, hipStream_t s) {
   const size_t shm = sizeof(float) * (size_t)nb.cap * 6;
-  hipLaunchKernelGGL(k_density_factor_t, dim3(nbricks(g)), dim3(PB), shm, s, make_args(c, g, gb, f, b, nb), f.rho,
-                     f.alpha, f.s, f.badv, f.kappav, div_warm, divergence_on, aux);
+  hipLaunchKernelGGL(k_density_factor_t, dim3(nbricks(g)), dim3(PB), shm, s, whole_bricks(make_args(c, g, gb, f, b, nb)),
+                     f.rho, f.alpha, f.s, f.badv, f.kappav, div_warm, divergence_on, aux);
 }
 
 void launch_velocity_update_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidBufs& f, BoundaryBufs& b,
                               NbrBufs& nb, RigidDev* rig, const float* kfield, float* kappa_acc, hipStream_t s,
                               const int* stop, IterTapeOut tape) {
   const size_t shm = sizeof(float) * (size_t)nb.cap * 4;
-  hipLaunchKernelGGL(k_velocity_update_t, dim3(nbricks(g)), dim3(VB), shm, s, make_args(c, g, gb, f, b, nb), kfield,
-                     kappa_acc, rig, stop, tape);
+  const PassArgs a = make_args(c, g, gb, f, b, nb);
+  const dim3 grid(pass_grid(g, nb.parts_log2));
+  constexpr int V1 = velocity_block<1>(), V4 = velocity_block<4>();
+  if (nb.parts_log2 > 0)
+    hipLaunchKernelGGL((k_velocity_update_t<4, V4>), grid, dim3(V4), shm, s, a, kfield, kappa_acc, rig, stop, tape);
+  else
+    hipLaunchKernelGGL((k_velocity_update_t<1, V1>), grid, dim3(V1), shm, s, a, kfield, kappa_acc, rig, stop, tape);
 }
 
 void launch_recompute_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidBufs& f, BoundaryBufs& b,
                         NbrBufs& nb, int mode, float kcoef, double* err_slot, hipStream_t s, const float* kpred,
                         const int* stop) {
   const size_t shm = sizeof(float) * (size_t)nb.cap * 6;
-  hipLaunchKernelGGL(k_recompute_t, dim3(nbricks(g)), dim3(PB), shm, s, make_args(c, g, gb, f, b, nb), mode, kcoef,
-                     f.rho, f.alpha, f.badv, f.kf, f.kappa, err_slot, kpred, stop);
+  hipLaunchKernelGGL(nb.parts_log2 > 0 ? k_recompute_t<4> : k_recompute_t<1>, dim3(pass_grid(g, nb.parts_log2)),
+                     dim3(PB), shm, s, make_args(c, g, gb, f, b, nb), mode, kcoef, f.rho, f.alpha, f.badv, f.kf,
+                     f.kappa, err_slot, kpred, stop);
 }
 
 void launch_expand_lists(const GridDesc& g, GridBufs& gb, FluidBufs& f, NbrBufs& nb, uint32_t* out, hipStream_t s) {
@@ -638,11 +910,13 @@ void launch_expand_lists(const GridDesc& g, GridBufs& gb, FluidBufs& f, NbrBufs&
 
 void set_tiled_kernel_attributes() {
   const int shm6 = (int)(sizeof(float) * TILE_CAP * 6), shm4 = (int)(sizeof(float) * TILE_CAP * 4);
-  (void)hipFuncSetAttribute((const void*)k_density_factor_t, hipFuncAttributeMaxDynamicSharedMemorySize, shm6);
-  (void)hipFuncSetAttribute((const void*)k_recompute_t, hipFuncAttributeMaxDynamicSharedMemorySize, shm6);
-  (void)hipFuncSetAttribute((const void*)k_velocity_update_t, hipFuncAttributeMaxDynamicSharedMemorySize, shm4);
-  (void)hipFuncSetAttribute((const void*)k_build_tiled, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)(sizeof(float) * 3 * BSTRIDE));
+  for (const void* k : {(const void*)k_density_factor_t, (const void*)k_recompute_t<1>, (const void*)k_recompute_t<4>})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, shm6);
+  for (const void* k : {(const void*)k_velocity_update_t<1, velocity_block<1>()>,
+                        (const void*)k_velocity_update_t<4, velocity_block<4>()>})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, shm4);
+  for (const void* k : {(const void*)k_build_tiled, (const void*)k_build_cells})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(float) * 3 * BSTRIDE));
 }
 
 }  // namespace dfr
