@@ -1765,6 +1765,7 @@ int dfr_init(dfr_ctx* c) {
     c->gb.fcount = dalloc<uint32_t>(c, nk); c->gb.fstart = dalloc<uint32_t>(c, nk + 1);
     c->gb.bcount = dalloc<uint32_t>(c, nk); c->gb.bstart = dalloc<uint32_t>(c, nk + 1);
     c->gb.key = dalloc<uint32_t>(c, NF); c->gb.slot = dalloc<uint32_t>(c, NF); c->gb.perm = dalloc<uint32_t>(c, NF);
+    c->gb.ent = dalloc<uint4>(c, NF); c->gb.bent = dalloc<uint4>(c, NB);
     c->gb.bkey = dalloc<uint32_t>(c, NB); c->gb.bslot = dalloc<uint32_t>(c, NB); c->gb.bperm = dalloc<uint32_t>(c, NB);
     c->gb.tile_sums = dalloc<uint32_t>(c, 2 * (scan_tile_count(nk) + 1));
     // the sorts expect zero counts and leave them zero

@@ -16,7 +16,7 @@ namespace dfr {
 // Cell key and a slot within the cell.  The fluid arrives in the previous
 // step's cell order, so a wavefront's keys form runs of equal values; each run
 // takes its slots with one atomic (the leader's), the other lanes add their
-// rank in the run.  Slot order within a cell is then fixed by k_cell_sort.
+// rank in the run.  The order within a cell is then fixed by k_place.
 // The fluid and the boundary samples are sorted by the same launches: the
 // blocks of a grid over particles split at S.split between the two sets, the
 // per-cell kernels take the set from blockIdx.y.
@@ -52,85 +52,42 @@ __global__ void k_keys(SortSets S, GridDesc g) {
   if (valid) T.slot[i] = base + (uint32_t)(lane - first);
 }
 
+// Index, order key (particle id for the fluid, sample index for the boundary)
+// and cell range of every entry, at its slot of the cell.
 __global__ void k_scatter(SortSets S) {
   uint32_t lb;
   const SortSet& T = set_of_block(S, xcd_block(), lb);
   const uint32_t i = lb * blockDim.x + threadIdx.x;
   if (i >= T.n) return;
-  T.perm[T.start[T.key[i]] + T.slot[i]] = i;
+  const uint32_t c = T.key[i];
+  const uint32_t s = T.start[c], e = T.start[c + 1];
+  T.ent[s + T.slot[i]] = make_uint4(i, T.order ? T.order[i] : i, s, e);
 }
 
-// Sort of each cell's entries by an order key (particle id for the fluid,
-// sample index for the boundary; keys are unique, so the result does not
-// depend on the slot order k_keys produced).  Cells hold about ten particles:
-// up to 16 entries are loaded together and sorted in registers by a bitonic
-// network; larger cells use an insertion sort.
-constexpr int CELL_NET = 16;
-__global__ void k_cell_sort(SortSets S, uint32_t nkeys) {
-  const SortSet& T = S.s[blockIdx.y];
-  const uint32_t* __restrict__ start = T.start;
-  uint32_t* __restrict__ perm = T.perm;
-  const uint32_t* __restrict__ order = T.order;
-  const uint32_t c = gid();
-  if (c >= nkeys) return;
-  const uint32_t s = start[c], e = start[c + 1];
-  const uint32_t m = e - s;
-  if (m < 2) return;
-  if (m <= (uint32_t)CELL_NET) {
-    uint32_t v[CELL_NET], kv[CELL_NET];
-#pragma unroll
-    for (int a = 0; a < CELL_NET; ++a) v[a] = ((uint32_t)a < m) ? perm[s + a] : 0u;
-#pragma unroll
-    for (int a = 0; a < CELL_NET; ++a) kv[a] = ((uint32_t)a < m) ? (order ? order[v[a]] : v[a]) : 0xffffffffu;
-#pragma unroll
-    for (int kk = 2; kk <= CELL_NET; kk <<= 1)
-#pragma unroll
-      for (int j = kk >> 1; j > 0; j >>= 1)
-#pragma unroll
-        for (int a = 0; a < CELL_NET; ++a) {
-          const int b = a ^ j;
-          if (b > a) {
-            const bool asc = (a & kk) == 0;
-            const bool sw = asc ? (kv[a] > kv[b]) : (kv[a] < kv[b]);
-            const uint32_t ka = kv[a], kb = kv[b], va = v[a], vb = v[b];
-            kv[a] = sw ? kb : ka; kv[b] = sw ? ka : kb;
-            v[a] = sw ? vb : va; v[b] = sw ? va : vb;
-          }
-        }
-#pragma unroll
-    for (int a = 0; a < CELL_NET; ++a)
-      if ((uint32_t)a < m) perm[s + a] = v[a];
-    return;
-  }
-  for (uint32_t a = s + 1; a < e; ++a) {
-    const uint32_t v = perm[a];
-    const uint32_t kv = order ? order[v] : v;
-    uint32_t b = a;
-    while (b > s) {
-      const uint32_t u = perm[b - 1];
-      const uint32_t ku = order ? order[u] : u;
-      if (ku <= kv) break;
-      perm[b] = u;
-      --b;
-    }
-    perm[b] = v;
-  }
-}
-
-// Permute the per-particle fluid state into sorted order.
-__global__ void k_gather_fluid(int n, const uint32_t* __restrict__ perm, const float4* __restrict__ pos,
-                               const float4* __restrict__ vel, const float* __restrict__ kappa,
-                               const float* __restrict__ kappav, const uint32_t* __restrict__ id,
-                               float4* __restrict__ pos2, float4* __restrict__ vel2, float* __restrict__ kappa2,
-                               float* __restrict__ kappav2, uint32_t* __restrict__ id2) {
-  const uint32_t k = gid();
-  if (k >= (uint32_t)n) return;
-  const uint32_t i = perm[k];
-  pos2[k] = pos[i];
-  vel2[k] = vel[i];
-  kappa2[k] = kappa[i];
-  kappav2[k] = kappav[i];
-  id2[k] = id[i];
+// Places every entry of a cell by its rank among the cell's order keys (unique,
+// so the result does not depend on the slot order k_keys produced) and moves the
+// fluid's state along.  One thread per entry: the entries of a cell are
+// consecutive, so the lanes of a wavefront compare against the same ten to
+// twenty keys.  One thread per cell, sorting its entries in registers (16 and
+// less) or in place, cost its longest chain whatever the scene's size: 17.5 us
+// at 8,000 particles, 32 at 250,000, 40 at 1M, and a launch of its own; this
+// makes the move 4.4, 7.2 and 22.8 us (3.8, 5.6 and 15.8 without the ranks).
+__global__ void k_place(SortSets S, FluidMove M) {
+  uint32_t lb;
+  const SortSet& T = set_of_block(S, xcd_block(), lb);
+  const uint32_t p = lb * blockDim.x + threadIdx.x;
+  if (p >= T.n) return;
+  const uint4 en = T.ent[p];
+  uint32_t to = en.z;
+#pragma unroll 4
+  for (uint32_t q = en.z; q < en.w; ++q) to += T.ent[q].y < en.y ? 1u : 0u;
+  T.perm[to] = en.x;
+  if (T.order == nullptr) return;  // the boundary samples stay where they are
+  M.pos2[to] = T.pos[en.x];
+  M.vel2[to] = M.vel[en.x];
+  M.kappa2[to] = M.kappa[en.x];
+  M.kappav2[to] = M.kappav[en.x];
+  M.id2[to] = en.y;
 }
 
 // ---------------------------------------------------------------------------
@@ -267,7 +224,7 @@ size_t scan_tile_count(uint32_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }
 
 // Sorts the sets of S (nsets = 1 or 2) by cell.  The counts must be zero on
 // entry (they are left zero).
-static void launch_sort_sets(const SortSets& S, int nsets, const GridDesc& g, hipStream_t s) {
+static void launch_sort_sets(const SortSets& S, int nsets, const FluidMove& M, const GridDesc& g, hipStream_t s) {
   const uint32_t nk = g.nkeys;
   const unsigned particle_blocks = S.split + (nsets > 1 ? blocks_for(S.s[1].n) : 0u);
   const unsigned tiles = (unsigned)scan_tile_count(nk);
@@ -277,15 +234,15 @@ static void launch_sort_sets(const SortSets& S, int nsets, const GridDesc& g, hi
   hipLaunchKernelGGL(k_scan_add, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk);
   if (particle_blocks) {
     hipLaunchKernelGGL(k_scatter, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S);
-    hipLaunchKernelGGL(k_cell_sort, dim3(blocks_for(nk), nsets), dim3(DFR_BLOCK), 0, s, S, nk);
+    hipLaunchKernelGGL(k_place, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S, M);
   }
 }
 
 static SortSet fluid_set(FluidBufs& f, GridBufs& gb) {
-  return SortSet{f.pos, (uint32_t)f.n, gb.fcount, gb.key, gb.slot, gb.fstart, gb.perm, f.id, gb.tile_sums};
+  return SortSet{f.pos, (uint32_t)f.n, gb.fcount, gb.key, gb.slot, gb.fstart, gb.ent, gb.perm, f.id, gb.tile_sums};
 }
 static SortSet boundary_set(BoundaryBufs& b, GridBufs& gb, uint32_t nk) {
-  return SortSet{b.pos, (uint32_t)b.n, gb.bcount, gb.bkey, gb.bslot, gb.bstart, gb.bperm, nullptr,
+  return SortSet{b.pos, (uint32_t)b.n, gb.bcount, gb.bkey, gb.bslot, gb.bstart, gb.bent, gb.bperm, nullptr,
                  gb.tile_sums + scan_tile_count(nk) + 1};
 }
 
@@ -295,19 +252,15 @@ void launch_sort_fluid_and_boundary(FluidBufs& f, BoundaryBufs& b, const GridDes
   S.s[0] = fluid_set(f, gb);
   S.s[1] = boundary_set(b, gb, g.nkeys);
   S.split = blocks_for(S.s[0].n);
-  launch_sort_sets(S, 2, g, s);
-  if (f.n > 0) {
-    hipLaunchKernelGGL(k_gather_fluid, dim3(blocks_for(f.n)), dim3(DFR_BLOCK), 0, s, f.n, gb.perm, f.pos, f.vel,
-                       f.kappa, f.kappav, f.id, f.pos2, f.vel2, f.kappa2, f.kappav2, f.id2);
-    f.swap_sorted();
-  }
+  launch_sort_sets(S, 2, FluidMove{f.vel, f.kappa, f.kappav, f.pos2, f.vel2, f.kappa2, f.kappav2, f.id2}, g, s);
+  if (f.n > 0) f.swap_sorted();
 }
 
 void launch_sort_boundary(BoundaryBufs& b, const GridDesc& g, GridBufs& gb, hipStream_t s) {
   SortSets S{};
   S.s[0] = boundary_set(b, gb, g.nkeys);
   S.split = blocks_for(S.s[0].n);
-  launch_sort_sets(S, 1, g, s);
+  launch_sort_sets(S, 1, FluidMove{}, g, s);
 }
 
 void launch_build_bf(FluidBufs& f, BoundaryBufs& b, const GridDesc& g, GridBufs& gb, NbrBufs& nb, float h2,

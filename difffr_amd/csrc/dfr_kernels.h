@@ -50,6 +50,7 @@ struct GridBufs {
   uint32_t *fcount = nullptr, *fstart = nullptr, *bcount = nullptr, *bstart = nullptr;
   uint32_t *key = nullptr, *slot = nullptr, *perm = nullptr;
   uint32_t *bkey = nullptr, *bslot = nullptr, *bperm = nullptr;
+  uint4 *ent = nullptr, *bent = nullptr;  // entries by cell, before their order in it
   uint32_t* tile_sums = nullptr;
 };
 
@@ -89,7 +90,8 @@ int gather_parts_log2(int nf);
 // dfr_grid.hip
 size_t scan_tile_count(uint32_t n);
 // One index set of the cell sort: positions, per-cell counts (zero between
-// sorts), cell key and slot of each index, cell starts (nkeys + 1), the
+// sorts), cell key and slot of each index, cell starts (nkeys + 1), the entries by
+// cell (index, order key, cell range), the
 // permutation, the in-cell order key (nullptr: the index itself) and
 // scan_tile_count(nkeys) + 1 words of scan scratch.
 struct SortSet {
@@ -99,9 +101,17 @@ struct SortSet {
   uint32_t* key;
   uint32_t* slot;
   uint32_t* start;
+  uint4* ent;
   uint32_t* perm;
   const uint32_t* order;
   uint32_t* tile_sums;
+};
+struct FluidMove {  // the fluid's state besides positions and ids, and where the sort puts all of it
+  const float4* vel;
+  const float *kappa, *kappav;
+  float4 *pos2, *vel2;
+  float *kappa2, *kappav2;
+  uint32_t* id2;
 };
 struct SortSets {
   SortSet s[2];
