@@ -34,14 +34,14 @@ struct PairCE {
 __device__ inline PairCE cubic_ce(const KernelConst& K, float r2, bool on = true) {
   const float irl = __builtin_amdgcn_rsqf(r2);
   const float q = r2 * irl * K.inv_h;
-  const float f = 1.f - q;
+  const float f = unit(1.f - q);
   const bool inner = q <= 0.5f;
   const float cin = fmaf(q, 3.f * K.l_ih2, -2.f * K.l_ih2);
   const float g = (f * f) * (K.l_ih * irl);
   const float cout = -g;
   const float ein = (3.f * K.l_ih2 * K.inv_h) * irl;
   const float eout = fmaf(2.f * K.l_ih2, f, g) * (irl * irl);
-  const bool valid = on && r2 > 1.0e-10f && q <= 1.f;
+  const bool valid = on && r2 > 1.0e-10f;
   PairCE o;
   o.c = valid ? (inner ? cin : cout) : 0.f;
   o.e = valid ? (inner ? ein : eout) : 0.f;

@@ -119,16 +119,21 @@ __device__ inline PairKernel cubic_pair(const KernelConst& K, float r2, bool on 
   o.c = (on && r2 > 1.0e-10f && !far) ? (inner ? cin : cout) : 0.f;
   return o;
 }
+// x clamped to [0, 1]: an output modifier of the instruction that makes x.
+__device__ inline float unit(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, 1.f); }
+// Beyond the support 1 - q clamps to 0 and so does the outer branch, so the pair
+// loops, bound by their vector instructions, test no q <= 1 (1M particles:
+// recompute 54.4 -> 52.7 us, velocity update 41.8 -> 40.4).
 // on = false gives 0 (a pair that contributes nothing), folded into the
 // support test's select.
 __device__ inline float cubic_grad_c(const KernelConst& K, float r2, bool on = true) {
   const float irl = __builtin_amdgcn_rsqf(r2);
   const float q = r2 * irl * K.inv_h;
-  const float f = 1.f - q;
+  const float f = unit(1.f - q);
   const float cin = fmaf(q, 3.f * K.l_ih2, -2.f * K.l_ih2);
   const float cout = -K.l_ih * (f * f) * irl;
   const float cc = (q <= 0.5f) ? cin : cout;
-  return (on && r2 > 1.0e-10f && q <= 1.f) ? cc : 0.f;
+  return (on && r2 > 1.0e-10f) ? cc : 0.f;
 }
 
 // gradGradW(r) = a * I + b * r r^T (SPHKernels.h:122-149 rewritten with
