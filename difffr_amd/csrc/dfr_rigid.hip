@@ -170,104 +170,108 @@ __device__ inline M3d grad_inertia_v(const RigidDev& b, const M3d& R, const M3d&
   return a + c;
 }
 
-__device__ void chain_rule(RigidDev& b, const RigidStepConst& rc) {
+// The Jacobians with respect to v0 and omega0 only ever take products from the
+// left, so each of their six columns goes by itself: lane c of the body's
+// wavefront carries column c (0..2 of v0, 3..5 of omega0).  One thread with
+// whole matrices was some 1,500 FP64 instructions of straight-line code and cost
+// their fetch: 40 us a step with one body (34 to 45), 6.5 by columns.
+struct V4d { double a[4]; };
+__device__ inline V3d col3(const double* p, int c) { return {p[c], p[3 + c], p[6 + c]}; }
+__device__ inline void put3(double* p, int c, V3d v) { p[c] = v.x; p[3 + c] = v.y; p[6 + c] = v.z; }
+__device__ inline V3d mv4(const M34d& A, const V4d& v) {
+  double o[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t += A(r, k) * v.a[k];
+    o[r] = t;
+  }
+  return {o[0], o[1], o[2]};
+}
+__device__ inline V3d add(V3d a, V3d b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
+__device__ inline V3d axpy(V3d a, V3d b, double s) { return {a.x + b.x * s, a.y + b.y * s, a.z + b.z * s}; }
+__device__ inline V3d grad_inertia_column(const RigidDev& b, const M3d& R, const M3d& I0, V3d v, const V4d& jq) {
+  const V3d u = mv(I0, mv(R.tr(), v));
+  return add(mv4(grad_Rqp<double>(b.q, u, 1.0), jq), mv(R, mv(I0, mv4(grad_Rqp<double>(b.q, v, -1.0), jq))));
+}
+
+__device__ void chain_rule(RigidDev& b, const RigidStepConst& rc, int c) {
   const double dt = rc.dt;
   const int mode = rc.gradient_mode;
   const double invMass = 1.0 / (b.mass + 1e-10);
   const M3d I = ld3(b.I), Iinv = ld3(b.Iinv), I0 = ld3(b.I0);
   const M3d R = quat_to_R(b.q);
   const V3d om = {b.w[0], b.w[1], b.w[2]};
-  M3d Jxv = ld3(b.J + 0), Jxw = ld3(b.J + 9), Jvv = ld3(b.J + 18), Jvw = ld3(b.J + 27), Jwv = ld3(b.J + 36),
-      Jww = ld3(b.J + 45);
-  M43d Jqv = ld43(b.J + 54), Jqw = ld43(b.J + 66);
-  const M3d nFv = ld3(b.net + 0), nFx = ld3(b.net + 9), nFw = ld3(b.net + 18), nTw = ld3(b.net + 27),
-            nTx = ld3(b.net + 36), nTv = ld3(b.net + 45);
-  const M34d nFq = ld34(b.net + 54), nTq = ld34(b.net + 66);
+  const bool w0 = c >= 3;
+  const int k = w0 ? c - 3 : c;
+  double *px = b.J + (w0 ? 9 : 0), *pv = b.J + (w0 ? 27 : 18), *pw = b.J + (w0 ? 45 : 36), *pq = b.J + (w0 ? 66 : 54);
+  V3d jx = col3(px, k), jv = col3(pv, k), jw = col3(pw, k);
+  V4d jq = {{pq[k], pq[3 + k], pq[6 + k], pq[9 + k]}};
   V3d temp = {0, 0, 0};
   const V3d Iom = mv(I, om);
+  // d((I w) x w) for this column
+  auto gyroscopic = [&]() {
+    return add(cross(Iom, jw), mv(skew(om).tr(), add(mv(I, jw), grad_inertia_column(b, R, I0, om, jq))));
+  };
+  // "+" on the d(I^-1) term as in the reference (:641-647)
+  auto spin = [&](V3d dTau) {
+    const V3d gI = mv(Iinv, grad_inertia_column(b, R, I0, mv(Iinv, temp), jq));
+    jw = axpy(jw, add(gI, mv(Iinv, dTau)), dt);
+  };
   if (mode == 0 || mode == 1) {
-    M3d dFv0, dFw0;
-    if (mode == 0) {
-      dFv0 = mm(nFx, Jxv) + mm(nFv, Jvv) + mm(nFq, Jqv) + mm(nFw, Jwv);
-      dFw0 = mm(nFx, Jxw) + mm(nFv, Jvw) + mm(nFq, Jqw) + mm(nFw, Jww);
-    } else {
-      dFv0 = mm(nFv, Jvv) + mm(nFw, Jwv);
-      dFw0 = mm(nFv, Jvw) + mm(nFw, Jww);
-    }
-    Jvv = Jvv + dFv0 * (dt * invMass);
-    Jvw = Jvw + dFw0 * (dt * invMass);
-    Jxv = Jxv + Jvv * dt;
-    Jxw = Jxw + Jvw * dt;
-    const V3d T = {b.T[0], b.T[1], b.T[2]};
-    M3d dTw0, dTv0;
-    if (mode == 0) {
-      dTw0 = mm(nTx, Jxw) + mm(nTv, Jvw) + mm(nTq, Jqw) + mm(nTw, Jww);
-      dTv0 = mm(nTx, Jxv) + mm(nTv, Jvv) + mm(nTq, Jqv) + mm(nTw, Jwv);
-    } else {
-      dTw0 = mm(nTv, Jvw) + mm(nTw, Jww);
-      dTv0 = mm(nTv, Jvv) + mm(nTw, Jwv);
-    }
-    M3d dTauw0, dTauv0;
+    auto force = [&](int x, int v, int q, int w) {
+      const V3d vw = add(mv(ld3(b.net + v), jv), mv(ld3(b.net + w), jw));
+      return mode == 0 ? add(vw, add(mv(ld3(b.net + x), jx), mv4(ld34(b.net + q), jq))) : vw;
+    };
+    jv = axpy(jv, force(9, 0, 54, 18), dt * invMass);
+    jx = axpy(jx, jv, dt);
+    V3d dTau = force(36, 45, 66, 27);
+    temp = {b.T[0], b.T[1], b.T[2]};
     if (rc.gyroscopic) {
-      const V3d lw = cross(Iom, om);
-      temp = {lw.x + T.x, lw.y + T.y, lw.z + T.z};
-      const M3d dLw_w0 = mm(skew(Iom), Jww) + mm(skew(om).tr(), mm(I, Jww) + grad_inertia_v(b, R, I0, om, Jqw));
-      const M3d dLw_v0 = mm(skew(Iom), Jwv) + mm(skew(om).tr(), mm(I, Jwv) + grad_inertia_v(b, R, I0, om, Jqv));
-      dTauw0 = dLw_w0 + dTw0;
-      dTauv0 = dLw_v0 + dTv0;
-    } else {
-      temp = T;
-      dTauw0 = dTw0;
-      dTauv0 = dTv0;
+      temp = add(cross(Iom, om), temp);
+      dTau = add(gyroscopic(), dTau);
     }
-    // "+" on the d(I^-1) term as in the reference (:641-647)
-    const V3d it = mv(Iinv, temp);
-    const M3d gIw = mm(Iinv, grad_inertia_v(b, R, I0, it, Jqw));
-    const M3d gIv = mm(Iinv, grad_inertia_v(b, R, I0, it, Jqv));
-    Jww = Jww + (gIw + mm(Iinv, dTauw0)) * dt;
-    Jwv = Jwv + (gIv + mm(Iinv, dTauv0)) * dt;
+    spin(dTau);
   } else {
-    Jxv = Jxv + Jvv * dt;
-    Jxw = Jxw + Jvw * dt;
+    jx = axpy(jx, jv, dt);
     if (rc.gyroscopic) {
       temp = cross(Iom, om);
-      const V3d it = mv(Iinv, temp);
-      const M3d gIw = mm(Iinv, grad_inertia_v(b, R, I0, it, Jqw));
-      const M3d gIv = mm(Iinv, grad_inertia_v(b, R, I0, it, Jqv));
-      const M3d dLw_w0 = mm(skew(Iom), Jww) + mm(skew(om).tr(), mm(I, Jww) + grad_inertia_v(b, R, I0, om, Jqw));
-      const M3d dLw_v0 = mm(skew(Iom), Jwv) + mm(skew(om).tr(), mm(I, Jwv) + grad_inertia_v(b, R, I0, om, Jqv));
-      Jww = Jww + (gIw + mm(Iinv, dLw_w0)) * dt;
-      Jwv = Jwv + (gIv + mm(Iinv, dLw_v0)) * dt;
+      spin(gyroscopic());
     }
   }
   if (rc.optimize_rotation) {
     const V3d it = mv(Iinv, temp);
-    const double nw[3] = {om.x + it.x * dt, om.y + it.y * dt, om.z + it.z * dt};
-    const double p[4] = {0.0, nw[0], nw[1], nw[2]};
-    double pq[4];
-    quat_mul(p, b.q, pq);
-    double nq[4];
-    for (int k = 0; k < 4; ++k) nq[k] = b.q[k] + dt * 0.5 * pq[k];
+    const double p[4] = {0.0, om.x + it.x * dt, om.y + it.y * dt, om.z + it.z * dt};
+    double pqm[4], nq[4], qh[4];
+    quat_mul(p, b.q, pqm);
+    for (int m = 0; m < 4; ++m) nq[m] = b.q[m] + dt * 0.5 * pqm[m];
     const double nn = sqrt(nq[1] * nq[1] + nq[2] * nq[2] + nq[3] * nq[3] + nq[0] * nq[0]);
-    double qh[4];
-    for (int k = 0; k < 4; ++k) qh[k] = nq[k] / nn;
-    M4d Nq;
-    for (int r = 0; r < 4; ++r)
-      for (int cc = 0; cc < 4; ++cc) Nq(r, cc) = ((r == cc) ? 1.0 : 0.0) - qh[r] * qh[cc];
-    Nq = Nq * (1.0 / nn);
-    M4d Pq;
-    const double pv[16] = {p[0], -p[1], -p[2], -p[3], p[1], p[0], -p[3], p[2],
-                           p[2], p[3], p[0], -p[1], p[3], -p[2], p[1], p[0]};
-    for (int k = 0; k < 16; ++k) Pq.a[k] = pv[k];
-    M43d Pw;
+    for (int m = 0; m < 4; ++m) qh[m] = nq[m] / nn;
     const double* q = b.q;
-    const double wv[12] = {-q[1], -q[2], -q[3], q[0], q[3], -q[2], -q[3], q[0], q[1], q[2], -q[1], q[0]};
-    for (int k = 0; k < 12; ++k) Pw.a[k] = wv[k];
-    Jqw = mm(Nq, Jqw + (mm(Pw, Jww) + mm(Pq, Jqw)) * (dt / 2.0));
-    Jqv = mm(Nq, Jqv + (mm(Pw, Jwv) + mm(Pq, Jqv)) * (dt / 2.0));
+    const double Pq[16] = {p[0], -p[1], -p[2], -p[3], p[1], p[0], -p[3], p[2],
+                           p[2], p[3], p[0], -p[1], p[3], -p[2], p[1], p[0]};
+    const double Pw[12] = {-q[1], -q[2], -q[3], q[0], q[3], -q[2], -q[3], q[0], q[1], q[2], -q[1], q[0]};
+    double e[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double pw3 = Pw[3 * r] * jw.x + Pw[3 * r + 1] * jw.y + Pw[3 * r + 2] * jw.z;
+      const double pq4 = Pq[4 * r] * jq.a[0] + Pq[4 * r + 1] * jq.a[1] + Pq[4 * r + 2] * jq.a[2] + Pq[4 * r + 3] * jq.a[3];
+      e[r] = jq.a[r] + (pw3 + pq4) * (dt / 2.0);
+    }
+    // (I - qh qh^T) / nn
+    V4d o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      double t = 0.0;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) t += (((r == m) ? 1.0 : 0.0) - qh[r] * qh[m]) * (1.0 / nn) * e[m];
+      o.a[r] = t;
+    }
+    jq = o;
   }
-  st3(b.J + 0, Jxv); st3(b.J + 9, Jxw); st3(b.J + 18, Jvv); st3(b.J + 27, Jvw); st3(b.J + 36, Jwv);
-  st3(b.J + 45, Jww); st43(b.J + 54, Jqv); st43(b.J + 66, Jqw);
+  put3(px, k, jx); put3(pv, k, jv); put3(pw, k, jw);
+  for (int r = 0; r < 4; ++r) pq[3 * r + k] = jq.a[r];
 }
 
 // RigidBodyGradientManager (single-body entries R == RR; no rigid contact).
@@ -340,26 +344,30 @@ __device__ void manager_position_chain(RigidDev& b, const RigidStepConst& rc) { 
 __device__ void rigid_forces(RigidDev& b, const RigidStepConst& rc);
 __device__ void rigid_animate(RigidDev& b, const RigidStepConst& rc);
 
-__global__ void k_rigid_step(RigidStepConst rc, RigidDev* __restrict__ rig) {
-  const int bi = threadIdx.x;
-  if (bi >= rc.nbodies) return;
+// One wavefront per body: lanes 0..5 the chain rule's columns, lane 0 the rest.
+__global__ void __launch_bounds__(64) k_rigid_step(RigidStepConst rc, RigidDev* __restrict__ rig) {
+  const int bi = blockIdx.x, lane = threadIdx.x;
   RigidDev& b = rig[bi];
   if (!b.dynamic) return;
   const int ph = rc.phases ? rc.phases : (RS_HAND | RS_MGR_VEL | RS_FORCES | RS_MGR_POS | RS_ANIMATE);
-  if ((ph & RS_HAND) && rc.compute_gradient && !b.animated) {
-    if (rc.use_manager) {
+  const bool hand = (ph & RS_HAND) && rc.compute_gradient && !b.animated;
+  if (hand && !rc.use_manager && lane < 6) chain_rule(b, rc, lane);
+  __syncthreads();  // the columns have read the body before lane 0 moves it
+  if (lane == 0) {
+    if (hand && rc.use_manager) {
       // update_rigid_body_gradient_manager (:952-967): the (R, R) entry
       double* dst = rc.mgr_net ? rc.mgr_net + ((size_t)bi * rc.nbodies + bi) * 78 : b.mnet;
       for (int k = 0; k < 78; ++k) dst[k] = b.net[k];
-    } else {
-      chain_rule(b, rc);
     }
+    // the manager's chain runs for every dynamic body (SimulatorBase.cpp:1159-1166)
+    if ((ph & RS_MGR_VEL) && rc.compute_gradient && rc.use_manager) manager_velocity_chain(b, rc);
+    if (ph & RS_FORCES) rigid_forces(b, rc);
+    if ((ph & RS_MGR_POS) && rc.compute_gradient && rc.use_manager) manager_position_chain(b, rc);
+    if (ph & RS_ANIMATE) rigid_animate(b, rc);
   }
-  // the manager's chain runs for every dynamic body (SimulatorBase.cpp:1159-1166)
-  if ((ph & RS_MGR_VEL) && rc.compute_gradient && rc.use_manager) manager_velocity_chain(b, rc);
-  if (ph & RS_FORCES) rigid_forces(b, rc);
-  if ((ph & RS_MGR_POS) && rc.compute_gradient && rc.use_manager) manager_position_chain(b, rc);
-  if (ph & RS_ANIMATE) rigid_animate(b, rc);
+  __syncthreads();
+  if (ph & RS_ANIMATE)
+    for (int k = lane; k < 78; k += 64) { b.netlast[k] = b.net[k]; b.net[k] = 0.0; }
 }
 
 // updateBoundaryForces and gravity (or, after the contact solver, its later
@@ -414,7 +422,6 @@ __device__ void rigid_animate(RigidDev& b, const RigidStepConst& rc) {
   const M3d In = mm(mm(R, ld3(b.I0)), R.tr());
   st3(b.I, In);
   st3(b.Iinv, inverse3(In));
-  for (int k = 0; k < 78; ++k) { b.netlast[k] = b.net[k]; b.net[k] = 0.0; }
 }
 
 // ---------------------------------------------------------------------------
@@ -552,7 +559,7 @@ void launch_gradient(const StepConst& c, const GradConst& gc, FluidBufs& f, Boun
 }
 
 void launch_rigid_step(const RigidStepConst& rc, RigidDev* rig, hipStream_t s) {
-  hipLaunchKernelGGL(k_rigid_step, dim3(1), dim3(64), 0, s, rc, rig);
+  if (rc.nbodies > 0) hipLaunchKernelGGL(k_rigid_step, dim3((unsigned)rc.nbodies), dim3(64), 0, s, rc, rig);
 }
 
 void launch_boundary_transform(const uint32_t* idx, int n, BoundaryBufs& b, const RigidDev* rig, hipStream_t s) {
