@@ -1139,20 +1139,18 @@ void tape_swap_out(dfr_ctx* c) {
   if (!A.swapped) return;
   const int nf = c->f.n;
   const auto& o = A.own;
-  d2d(c, o.nbr8, (const uint4*)c->nb.nbr8, (size_t)NPACK * nf);
-  {
-    const size_t NB = (size_t)c->grid.bn[0] * c->grid.bn[1] * c->grid.bn[2];
-    d2d(c, o.thdr, (const uint4*)c->nb.thdr, NB);
-    d2d(c, o.tmap, (const uint32_t*)c->nb.tmap, NB * TILE_CAP);
-  }
-  d2d(c, o.nbrB, (const uint32_t*)c->nb.nbrB, (size_t)c->nb.maxb * nf);
-  d2d(c, o.cnt, (const uint32_t*)c->nb.cnt, (size_t)nf);
-  d2d(c, o.fstart, (const uint32_t*)c->gb.fstart, (size_t)c->grid.nkeys + 1);
-  d2d(c, o.perm, (const uint32_t*)c->gb.perm, (size_t)nf);
-  d2d(c, o.rho, (const float*)c->f.rho, (size_t)nf);
-  d2d(c, o.alpha, (const float*)c->f.alpha, (size_t)nf);
-  d2d(c, o.s, (const float4*)c->f.s, (size_t)nf);
-  if (o.aux) d2d(c, o.aux, (const float2*)c->mlp.aux, (size_t)nf);
+  if (nf > 0)
+    launch_copy_lists(ListBufs{o.nbr8, o.thdr, o.tmap, o.nbrB, o.cnt},
+                      ListBufs{c->nb.nbr8, c->nb.thdr, c->nb.tmap, c->nb.nbrB, c->nb.cnt}, nf, c->nb.maxb, c->grid,
+                      c->stream);
+  Batch bt(c);
+  bt.copy(o.fstart, c->gb.fstart, (size_t)c->grid.nkeys + 1);
+  bt.copy(o.perm, c->gb.perm, (size_t)nf);
+  bt.copy(o.rho, c->f.rho, (size_t)nf);
+  bt.copy(o.alpha, c->f.alpha, (size_t)nf);
+  bt.copy(o.s, c->f.s, (size_t)nf);
+  if (o.aux) bt.copy(o.aux, c->mlp.aux, (size_t)nf);
+  bt.flush();
   c->nb.nbr8 = o.nbr8; c->nb.thdr = o.thdr; c->nb.tmap = o.tmap; c->nb.nbrB = o.nbrB; c->nb.cnt = o.cnt;
   c->gb.fstart = o.fstart; c->gb.perm = o.perm;
   c->f.rho = o.rho; c->f.alpha = o.alpha; c->f.s = o.s; c->mlp.aux = o.aux;

@@ -173,6 +173,13 @@ void launch_velocity_update_t(const StepConst& c, const GridDesc& g, GridBufs& g
 void launch_recompute_t(const StepConst& c, const GridDesc& g, GridBufs& gb, FluidBufs& f, BoundaryBufs& b,
                         NbrBufs& nb, int mode, float kcoef, double* err_slot, hipStream_t s,
                         const float* kpred = nullptr, const int* stop = nullptr);
+// A step's neighbour lists (NbrBufs' buffers of the same names).
+struct ListBufs {
+  uint4 *nbr8, *thdr;
+  uint32_t *tmap, *nbrB, *cnt;
+};
+void launch_copy_lists(const ListBufs& d, const ListBufs& src, int n, int maxb, const GridDesc& g,
+                       hipStream_t s);
 void launch_expand_lists(const GridDesc& g, GridBufs& gb, FluidBufs& f, NbrBufs& nb, uint32_t* out, hipStream_t s);
 void set_tiled_kernel_attributes();
 
