@@ -74,6 +74,21 @@ __global__ void k_boundary_volume(const float4* __restrict__ bpos_in, const floa
   bpos_out[j] = o;
 }
 
+// A field of the sorted particles at its place in id order (xyz of a float4).
+__global__ void k_export3(int n, const uint32_t* __restrict__ id, const float4* __restrict__ src,
+                          float* __restrict__ out) {
+  const uint32_t i = gid();
+  if (i >= (uint32_t)n) return;
+  const float4 v = src[i];
+  float* o = out + 3 * (size_t)id[i];
+  o[0] = v.x; o[1] = v.y; o[2] = v.z;
+}
+__global__ void k_export1(int n, const uint32_t* __restrict__ id, const float* __restrict__ src,
+                          float* __restrict__ out) {
+  const uint32_t i = gid();
+  if (i < (uint32_t)n) out[id[i]] = src[i];
+}
+
 // One Jacobi iteration's convergence test (divergenceSolve :816-828,
 // pressureSolve :700-712): continue while (avg > eta or it + 1 < min) and
 // it + 1 < max.  probe is host-visible memory.
@@ -145,6 +160,13 @@ void launch_solve_check(const double* part, int nparts, double* err, int n, doub
                         int max_it, int* stop, SolveProbe* probe, hipStream_t s) {
   hipLaunchKernelGGL(k_solve_check, dim3(1), dim3(CHECK_BLOCK), 0, s, part, nparts, err, n, eta, it, min_it, max_it,
                      stop, probe);
+}
+
+void launch_export_field(int n, const uint32_t* id, const float4* src, float* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_export3, dim3(nblk(n)), dim3(DFR_BLOCK), 0, s, n, id, src, out);
+}
+void launch_export_field(int n, const uint32_t* id, const float* src, float* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_export1, dim3(nblk(n)), dim3(DFR_BLOCK), 0, s, n, id, src, out);
 }
 
 void launch_advect(const StepConst& c, FluidBufs& f, float kappav_scale, hipStream_t s) {
