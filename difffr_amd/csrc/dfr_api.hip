@@ -972,8 +972,8 @@ void do_step(dfr_ctx* c) {
 // Per-particle fields in id order: reordered on the device into the context's
 // export buffer, then one copy into the caller's memory.  Bound by that copy.  A
 // copy of the sorted field, one of the ids and a host loop made a frame of
-// 250,000 particles (four steps, positions, velocities and density) 2584 us; 2023
-// this way.
+// 250,000 particles (three steps, positions and velocities) 2584 us; 2023 this
+// way.
 struct OnDevice {  // the context's device for a getter, which leaves the caller's current one as it was
   int prev = 0;
   explicit OnDevice(int device) {

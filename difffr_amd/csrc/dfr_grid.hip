@@ -94,8 +94,8 @@ __global__ void k_place(SortSets S, FluidMove M) {
 // Exclusive scan of the per-cell counts of each set (blockIdx.y): two passes, 2048
 // keys per block.  Every block of the second pass sums the tiles before its own
 // (a few hundred words at most) in place of a launch between the two, which cost
-// 2.2 to 3 us and its gap: ten steps with their reverse at 250,000 particles
-// 8080 -> 8027 us.  The second pass also clears the counts for the next sort.
+// 2.2 to 3 us and its gap: six checkpointed steps with their reverse at
+// 250,000 particles 8080 -> 8027 us.  The second pass also clears the counts for the next sort.
 // ---------------------------------------------------------------------------
 constexpr int SCAN_ITEMS = 8;
 constexpr int SCAN_TILE = DFR_BLOCK * SCAN_ITEMS;

@@ -860,8 +860,8 @@ k_expand_lists(GridDesc g, const uint32_t* __restrict__ fstart, int nf, const ui
 // brick for the maps; bound by memory.  Whole buffers hold 64 fluid slots and
 // maxb boundary samples a particle and 2,560 map entries a brick, some 500 MB at
 // 1M particles; the entries in use take 40 us there (250,000: 14.5), and a pass of
-// four recorded steps with their reverse went from 8454 to 8284 us (ten steps at
-// 250,000: 8167 to 8076).
+// four recorded steps with their reverse went from 8454 to 8284 us (six
+// checkpointed ones at 250,000: 8167 to 8076).
 __global__ void __launch_bounds__(DFR_BLOCK)
 k_copy_lists(ListBufs d, ListBufs s, uint32_t n, uint32_t maxb, uint32_t bricks, uint32_t particle_blocks) {
   if (blockIdx.x < particle_blocks) {
