@@ -1806,8 +1806,9 @@ int dfr_init(dfr_ctx* c) {
     HIPCHK(hipHostMalloc((void**)&c->h_overflow, sizeof(uint32_t) * 4, hipHostMallocDefault));
     c->h_overflow[0] = c->h_overflow[1] = c->h_overflow[2] = c->h_overflow[3] = 0;
     c->d_stop = dalloc<int>(c, 2);
-    c->nb.parts_log2 = gather_parts_log2(nf);
-    c->nparts = (int)(c->grid.bn[0] * c->grid.bn[1] * c->grid.bn[2]) << c->nb.parts_log2;
+    const uint32_t nbr = c->grid.bn[0] * c->grid.bn[1] * c->grid.bn[2];
+    c->nb.parts_log2 = gather_parts_log2(nf, nbr);
+    c->nparts = (int)(nbr << c->nb.parts_log2);
     c->d_part = dalloc<double>(c, c->nparts);
     c->probe_cap = std::max(c->P.max_iterations, c->P.max_iterations_v) + 1;
     HIPCHK(hipHostMalloc((void**)&c->h_probe, sizeof(SolveProbe) * 2 * c->probe_cap,

@@ -2,6 +2,7 @@
 #pragma once
 #include <utility>
 #include "dfr_device.h"
+#include "dfr_spread.h"
 
 namespace dfr {
 
@@ -68,24 +69,6 @@ struct NbrBufs {
   int cap = TILE_CAP;            // halo slots the passes stage in LDS; larger halos read global memory
   int parts_log2 = 0;            // workgroups per brick of the gather passes: 2^parts_log2 (gather_parts_log2)
 };
-
-// How a scene's gather passes are spread.  A pass of a few bricks costs the chain
-// of one wavefront: staging, then some 40 pairs one after the other per lane, and
-// up to 20 boundary samples a group at a time.  There, 2^parts workgroups share a
-// brick's particles (each stages the whole halo) and four lanes share a particle's
-// pairs.  The step's own passes still add in list order (Terms in dfr_tile.h): a
-// solve's masks flip on an ulp, and a trajectory would hang on the scene's size.
-// The reverse passes, linear in what they carry, add each lane's partial sum.
-// Measured, us a launch with one lane and one workgroup -> parts 2 (parts 1):
-//   particles   velocity            recompute           adjoint delta        adjoint div. update
-//     2,000     11.6 ->  7.2 (10.6) 10.5 ->  6.2 ( 9.2) 15.7 ->  6.7 (10.1)  20.7 ->  9.0 (12.4)
-//     8,500     14.9 ->  9.2 (10.8) 10.5 ->  7.9 ( 9.4) 16.4 ->  9.1 (10.9)  22.6 -> 11.1 (13.8)
-//    35,000     14.3 -> 10.8 (12.0) 11.9 ->  9.5 (10.5) 17.4 -> 11.6 (12.5)  20.6 -> 12.6 (13.6)
-//    56,000     15.2 -> 13.9 (17.0) 13.7 -> 15.3 (13.6) 21.4 -> 17.1 (17.3)  28.1 -> 19.1 (18.6)
-//    98,000     15.7 -> 19.7 (19.0) 15.7 -> 22.3 (18.4) 24.5 -> 27.3 (24.6)  25.5 -> 30.0 (25.6)
-// At 98,000 the chip is full with one workgroup a brick and the halo is staged
-// again for nothing.
-int gather_parts_log2(int nf);
 
 // dfr_grid.hip
 size_t scan_tile_count(uint32_t n);

@@ -887,10 +887,6 @@ k_copy_lists(ListBufs d, ListBufs s, uint32_t n, uint32_t maxb, uint32_t bricks,
 
 // ---------------------------------------------------------------------------
 
-int gather_parts_log2(int nf) {
-  return nf < 40000 ? 2 : nf < 80000 ? 1 : 0;
-}
-
 void launch_build_tiled(FluidBufs& f, BoundaryBufs& b, const GridDesc& g, GridBufs& gb, NbrBufs& nb, float h2,
                         hipStream_t s) {
   const size_t shm = sizeof(float) * 3 * (size_t)BSTRIDE;
