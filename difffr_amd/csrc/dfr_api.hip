@@ -383,6 +383,21 @@ GridDesc make_grid(const float lo_in[3], const float hi_in[3], float h) {
   return g;
 }
 
+// Bricks of the grid that hold some of the n particles.
+uint32_t filled_bricks(const GridDesc& g, const std::vector<float>& x, int64_t n) {
+  std::vector<bool> seen((size_t)g.bn[0] * g.bn[1] * g.bn[2]);
+  uint32_t filled = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    size_t b[3];
+    for (int k = 0; k < 3; ++k)
+      b[k] = (size_t)std::min(std::max((int)((x[3 * i + k] - g.lo[k]) * g.inv_cs), 0), g.n[k] - 1) / 4;
+    const size_t at = (b[2] * g.bn[1] + b[1]) * g.bn[0] + b[0];
+    filled += seen[at] ? 0u : 1u;
+    seen[at] = true;
+  }
+  return filled;
+}
+
 void fill_rigid_from_body(const dfr_ctx* c, const BodyInfo& bi, RigidDev& r) {
   std::memset(&r, 0, sizeof(r));
   for (int k = 0; k < 3; ++k) { r.x[k] = bi.x_rb[k]; r.v0[k] = bi.v0[k]; r.w0[k] = bi.w0[k]; }
@@ -1210,7 +1225,7 @@ void reverse_step(dfr_ctx* c, const StepTapeDev& T) {
   a.nbr8 = T.nbr8; a.thdr = T.thdr; a.tmap = T.tmap; a.nbrB = T.nbrB; a.cnt = T.cnt;
   a.bx = T.bpos; a.bv = T.bvel; a.bx0 = c->b.x0; a.nb_static = c->b.n - c->b.nd;
   a.cap = c->nb.cap;
-  a.parts_log2 = c->nb.parts_log2;
+  a.parts_log2 = c->nb.rev_parts_log2;
   a.sxb = A.sxb; a.svb = A.svb; a.body = A.body;
   {
     Timed t(c, TC_ADJ_MISC);
@@ -1807,7 +1822,10 @@ int dfr_init(dfr_ctx* c) {
     c->h_overflow[0] = c->h_overflow[1] = c->h_overflow[2] = c->h_overflow[3] = 0;
     c->d_stop = dalloc<int>(c, 2);
     const uint32_t nbr = c->grid.bn[0] * c->grid.bn[1] * c->grid.bn[2];
-    c->nb.parts_log2 = gather_parts_log2(nf, nbr);
+    c->nb.parts_log2 =
+        forward_parts_log2(nf, nbr, nf < FORWARD_PARTICLES ? filled_bricks(c->grid, c->fx, nf) : 0u);
+    c->nb.rev_parts_log2 = reverse_parts_log2(nf, nbr);
+    c->nb.by_cells = build_by_cells(nf, nbr);
     c->nparts = (int)(nbr << c->nb.parts_log2);
     c->d_part = dalloc<double>(c, c->nparts);
     c->probe_cap = std::max(c->P.max_iterations, c->P.max_iterations_v) + 1;

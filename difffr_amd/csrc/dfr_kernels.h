@@ -67,7 +67,9 @@ struct NbrBufs {
   uint32_t* overflow = nullptr;  // [4] max count seen when a list overflowed (fluid, B->F, boundary),
                                  //     largest halo of the last build
   int cap = TILE_CAP;            // halo slots the passes stage in LDS; larger halos read global memory
-  int parts_log2 = 0;            // workgroups per brick of the gather passes: 2^parts_log2 (gather_parts_log2)
+  int parts_log2 = 0;            // workgroups per brick of the step's spread passes: 2^parts_log2 (dfr_spread.h)
+  int rev_parts_log2 = 0;        // of the reverse passes
+  bool by_cells = false;         // lists by k_build_cells
 };
 
 // dfr_grid.hip

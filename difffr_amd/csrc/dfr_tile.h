@@ -227,7 +227,7 @@ __device__ inline void for_fluid_groups(const uint4* __restrict__ nbr8, size_t s
 }
 
 // The same with four lanes per particle, for the reverse passes (see
-// gather_parts_log2): lane l takes the slots 2 l and 2 l + 1 of each pack, two
+// dfr_spread.h): lane l takes the slots 2 l and 2 l + 1 of each pack, two
 // packs a round; the partial sums of the lanes are added at the end (lane_sum).
 template <int G, int L, class Load, class Body>
 __device__ inline void for_fluid_lanes(const uint4* __restrict__ nbr8, size_t stride, uint32_t i, uint32_t nF, int l,
@@ -291,7 +291,7 @@ __device__ inline void for_boundary_groups(const uint32_t* __restrict__ nbrB, si
 
 // ---------------------------------------------------------------------------
 // Four lanes per particle in the step's own passes (L = 4: small scenes, see
-// gather_parts_log2).  The lanes of a quad evaluate different pairs; every lane
+// dfr_spread.h).  The lanes of a quad evaluate different pairs; every lane
 // then adds all pairs' terms in list order, reading each from the lane that has
 // it (a quad broadcast costs one instruction), so the sums are those of one lane
 // per particle bit for bit.  `term` forms what a pair contributes (Terms), `acc`

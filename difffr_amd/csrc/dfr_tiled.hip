@@ -892,7 +892,7 @@ void launch_build_tiled(FluidBufs& f, BoundaryBufs& b, const GridDesc& g, GridBu
   const size_t shm = sizeof(float) * 3 * (size_t)BSTRIDE;
   // workgroups per brick of k_build_cells: 2,000 particles 17 us with 8, 21 with 4; 28,000: 41 and 35
   const int cell_parts_log2 = f.n < 16384 ? 3 : 2;
-  if (nb.parts_log2 > 0)
+  if (nb.by_cells)
     hipLaunchKernelGGL(k_build_cells, dim3(nbricks(g) << cell_parts_log2), dim3(BB), shm, s, f.pos, f.n, g, gb.fstart,
                        b.pos, gb.bstart, gb.bperm, h2, nb.maxb, nb.cap, cell_parts_log2, nb.nbr8, nb.nbrB, nb.cnt,
                        nb.overflow, nb.thdr, nb.tmap);
