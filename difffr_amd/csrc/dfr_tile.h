@@ -395,14 +395,22 @@ struct Slot8 {
 template <int L = 1, class Body>
 __device__ inline void for_fluid_slots_rolled(const uint4* __restrict__ nbr8, size_t stride, uint32_t i,
                                               uint32_t nF, Body&& body, int l = 0) {
-  constexpr uint32_t W = PACK / L;  // slots of a pack that a lane takes
+  if constexpr (L == 1) {
 #pragma unroll 1
-  for (uint32_t m = 0;; ++m) {
-    const uint32_t k = (m / W) * PACK + W * (uint32_t)l + m % W;
-    if ((m / W) * PACK >= nF) break;
-    if (k >= nF) continue;
-    const uint4 v = nbr8[(size_t)(k >> 3) * stride + i];
-    body(pack_get(v, (int)(k & 7u)));
+    for (uint32_t k = 0; k < nF; ++k) {
+      const uint4 v = nbr8[(size_t)(k >> 3) * stride + i];
+      body(pack_get(v, (int)(k & 7u)));
+    }
+  } else {
+    constexpr uint32_t W = PACK / L;  // slots of a pack that a lane takes
+#pragma unroll 1
+    for (uint32_t m = 0;; ++m) {
+      const uint32_t k = (m / W) * PACK + W * (uint32_t)l + m % W;
+      if ((m / W) * PACK >= nF) break;
+      if (k >= nF) continue;
+      const uint4 v = nbr8[(size_t)(k >> 3) * stride + i];
+      body(pack_get(v, (int)(k & 7u)));
+    }
   }
 }
 
