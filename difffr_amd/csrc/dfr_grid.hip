@@ -92,12 +92,17 @@ __global__ void k_place(SortSets S, FluidMove M) {
 
 // ---------------------------------------------------------------------------
 // Exclusive scan of the per-cell counts of each set (blockIdx.y): two passes, 2048
-// keys per block.  Every block of the second pass sums the tiles before its own
-// (a few hundred words at most) in place of a launch between the two, which cost
-// 2.2 to 3 us and its gap: six checkpointed steps with their reverse at
-// 250,000 particles 8080 -> 8027 us.  The second pass also clears the counts for the next sort.
+// keys per block.  Every block of the second pass sums the tiles before its own, in
+// place of a launch between the two, which cost 2.2 to 3 us and its gap: six
+// checkpointed steps with their reverse at 250,000 particles 8080 -> 8027 us.  That
+// is half the tile count squared in words: nothing for a tank (630 tiles at 4M
+// particles), 33 us at 22,800 tiles (46.7M cells), where the launch takes 71; 700 and
+// 200 at 63,000, 2,900 and 380 at 122,000.  So above SCAN_SUMS_TILES a launch of one
+// workgroup a set scans the tile sums (k_scan_sums).  The second pass also clears the
+// counts for the next sort.
 // ---------------------------------------------------------------------------
 constexpr int SCAN_ITEMS = 8;
+constexpr unsigned SCAN_SUMS_TILES = 32768;
 constexpr int SCAN_TILE = DFR_BLOCK * SCAN_ITEMS;
 
 __global__ void k_scan_tiles(SortSets S, uint32_t n) {
@@ -121,13 +126,35 @@ __global__ void k_scan_tiles(SortSets S, uint32_t n) {
   if (threadIdx.x == 0) T.tile_sums[blockIdx.x] = total;
 }
 
-__global__ void __launch_bounds__(DFR_BLOCK) k_scan_add(SortSets S, uint32_t n) {
+// Tile sums to the sums before each tile; the total goes past the last.
+__global__ void __launch_bounds__(DFR_BLOCK) k_scan_sums(SortSets S, uint32_t m) {
+  uint32_t* __restrict__ sums = S.s[blockIdx.x].tile_sums;
+  __shared__ uint32_t lds[DFR_BLOCK / 64 + 1];
+  uint32_t carry = 0;
+  for (uint32_t base = 0; base < m; base += DFR_BLOCK) {
+    const uint32_t i = base + threadIdx.x;
+    const uint32_t v = (i < m) ? sums[i] : 0u;
+    uint32_t total;
+    const uint32_t ex = block_exclusive_scan(v, lds, total);
+    if (i < m) sums[i] = ex + carry;
+    carry += total;
+  }
+  if (threadIdx.x == 0) sums[m] = carry;
+}
+
+__global__ void __launch_bounds__(DFR_BLOCK) k_scan_add(SortSets S, uint32_t n, int summed) {
   const SortSet& T = S.s[blockIdx.y];
   __shared__ uint32_t lds[DFR_BLOCK / 64 + 1];
-  uint32_t before = 0;
-  for (uint32_t m = threadIdx.x; m < blockIdx.x; m += DFR_BLOCK) before += T.tile_sums[m];
-  uint32_t add;
-  (void)block_exclusive_scan(before, lds, add);
+  uint32_t add, end;
+  if (summed) {
+    add = T.tile_sums[blockIdx.x];
+    end = T.tile_sums[blockIdx.x + 1];
+  } else {
+    uint32_t before = 0;
+    for (uint32_t m = threadIdx.x; m < blockIdx.x; m += DFR_BLOCK) before += T.tile_sums[m];
+    (void)block_exclusive_scan(before, lds, add);
+    end = add + T.tile_sums[blockIdx.x];
+  }
   const uint32_t base = blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
 #pragma unroll
   for (int k = 0; k < SCAN_ITEMS; ++k)
@@ -135,7 +162,7 @@ __global__ void __launch_bounds__(DFR_BLOCK) k_scan_add(SortSets S, uint32_t n) 
       T.start[base + k] += add;
       T.count[base + k] = 0u;
     }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) T.start[n] = add + T.tile_sums[blockIdx.x];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) T.start[n] = end;
 }
 
 // Fluid neighbours of the samples of dynamic bodies (the B->F lists the
@@ -221,7 +248,9 @@ static void launch_sort_sets(const SortSets& S, int nsets, const FluidMove& M, c
   const unsigned tiles = (unsigned)scan_tile_count(nk);
   if (particle_blocks) hipLaunchKernelGGL(k_keys, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S, g);
   hipLaunchKernelGGL(k_scan_tiles, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk);
-  hipLaunchKernelGGL(k_scan_add, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk);
+  const bool many = tiles > SCAN_SUMS_TILES;
+  if (many) hipLaunchKernelGGL(k_scan_sums, dim3(nsets), dim3(DFR_BLOCK), 0, s, S, tiles);
+  hipLaunchKernelGGL(k_scan_add, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk, (int)many);
   if (particle_blocks) {
     hipLaunchKernelGGL(k_scatter, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S);
     hipLaunchKernelGGL(k_place, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S, M);
