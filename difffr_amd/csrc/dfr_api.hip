@@ -1003,8 +1003,7 @@ template <typename T> void download_unpermute(const dfr_ctx* c, const T* src, fl
   const size_t words = (size_t)n * (sizeof(T) == sizeof(float4) ? 3 : 1);
   std::lock_guard<std::mutex> lock(c->export_mu);
   OnDevice dev(c->device);
-  launch_export_field(n, c->f.id, src, c->export_buf, c->stream);
-  HIPCHK(hipGetLastError());
+  HIPCHK(launch_export_field(n, c->f.id, src, c->export_buf, c->stream));
   HIPCHK(hipMemcpyAsync(out, c->export_buf, words * sizeof(float), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
 }

@@ -202,8 +202,8 @@ struct SolveProbe {
 void launch_solve_check(const double* part, int nparts, double* err, int n, double eta, int it, int min_it,
                         int max_it, int* stop, SolveProbe* probe, hipStream_t s);
 // Per-particle field to id order: 3 words of each float4, or 1.
-void launch_export_field(int n, const uint32_t* id, const float4* src, float* out, hipStream_t s);
-void launch_export_field(int n, const uint32_t* id, const float* src, float* out, hipStream_t s);
+hipError_t launch_export_field(int n, const uint32_t* id, const float4* src, float* out, hipStream_t s);
+hipError_t launch_export_field(int n, const uint32_t* id, const float* src, float* out, hipStream_t s);
 void launch_boundary_volume_impl(const float4* bpos_in, const float4* bx0, int nb, const int* groups, int nbodies,
                                  KernelConst K, float h2, const GridDesc& g, GridBufs& gb, float4* bpos_out,
                                  hipStream_t s);

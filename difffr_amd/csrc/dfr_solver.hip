@@ -162,11 +162,19 @@ void launch_solve_check(const double* part, int nparts, double* err, int n, doub
                      stop, probe);
 }
 
-void launch_export_field(int n, const uint32_t* id, const float4* src, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_export3, dim3(nblk(n)), dim3(DFR_BLOCK), 0, s, n, id, src, out);
+// hipLaunchKernel, whose own status says whether this launch was taken: the thread's
+// last error may be another call's.
+template <class T>
+static hipError_t export_field(void (*kernel)(int, const uint32_t*, const T*, float*), int n, const uint32_t* id,
+                               const T* src, float* out, hipStream_t s) {
+  void* args[] = {&n, &id, &src, &out};
+  return hipLaunchKernel((const void*)kernel, dim3(nblk(n)), dim3(DFR_BLOCK), args, 0, s);
 }
-void launch_export_field(int n, const uint32_t* id, const float* src, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_export1, dim3(nblk(n)), dim3(DFR_BLOCK), 0, s, n, id, src, out);
+hipError_t launch_export_field(int n, const uint32_t* id, const float4* src, float* out, hipStream_t s) {
+  return export_field(k_export3, n, id, src, out, s);
+}
+hipError_t launch_export_field(int n, const uint32_t* id, const float* src, float* out, hipStream_t s) {
+  return export_field(k_export1, n, id, src, out, s);
 }
 
 void launch_advect(const StepConst& c, FluidBufs& f, float kappav_scale, hipStream_t s) {
