@@ -3,10 +3,14 @@ sample counts around the kernel's groups of 16 samples a workgroup and 16
 lanes a sample: fewer, exactly and more than a group, with neighbour lists
 shorter and longer than 16, with and without the rotation entries.
 
-Tolerance: the sums hang on FP32 terms that cancel (b_i = rho* - 1), so the
-oracle's own FP32 and FP64 runs of the step differ by about 1e-3 of a block's
-largest entry; the GPU, which rounds like the FP32 run in another order, is
-held to three times the largest such spread of the blocks.
+Tolerance: the sums with respect to positions and rotations (F and T by x and q)
+hang on FP32 terms that cancel (b_i = rho* - 1), and the oracle's own FP32 and FP64
+runs of the step differ by 2e-4 to 1.6e-3 of a block's largest entry there; those
+with respect to velocities (by v and omega) have no such term and differ by 1e-7 to
+5e-6.  The GPU, which rounds like the FP32 run in another order, is held to three
+times the largest such spread of its kind of blocks (of at least 2e-6: some twenty
+FP32 operations a pair, 6e-8 each, and one unit more for the sum); the spreads
+themselves are held below 5e-3 and 1e-5, so neither bound can grow vacuous.
 """
 import numpy as np
 import pytest
@@ -17,7 +21,9 @@ from oracle.pyoracle import OracleSim
 
 pytestmark = pytest.mark.gpu
 
-BLOCKS = [(0, 9), (9, 18), (18, 27), (27, 36), (36, 45), (45, 54), (54, 66), (66, 78)]
+# (first, last, with respect to velocities)
+BLOCKS = [(0, 9, True), (9, 18, False), (18, 27, True), (27, 36, True), (36, 45, False), (45, 54, True),
+          (54, 66, False), (66, 78, False)]
 
 
 @pytest.mark.parametrize("samples,rotation", [(1, 1), (15, 1), (16, 0), (17, 1), (130, 1)])
@@ -43,10 +49,13 @@ def test_pair_sums_match_oracle(gpu_ready, samples, rotation):
         o.step(1)
         ref.append(o.net_gradients(1))
     blocks = BLOCKS if rotation else BLOCKS[:2]
-    scale = [np.abs(ref[0][lo:hi]).max() for lo, hi in blocks]
+    scale = [np.abs(ref[0][lo:hi]).max() for lo, hi, _ in blocks]
     assert min(scale) > 0.0
-    spread = max(np.abs(ref[0][lo:hi] - ref[1][lo:hi]).max() / s for (lo, hi), s in zip(blocks, scale))
-    for (lo, hi), s in zip(blocks, scale):
-        assert np.abs(ng[lo:hi] - ref[0][lo:hi]).max() <= 3.0 * spread * s, (lo, spread)
+    spread = {kind: max(np.abs(ref[0][lo:hi] - ref[1][lo:hi]).max() / s
+                        for (lo, hi, k), s in zip(blocks, scale) if k == kind) for kind in (True, False)}
+    assert spread[True] < 1e-5 and spread[False] < 5e-3, spread
+    spread[True] = max(spread[True], 2e-6)
+    for (lo, hi, kind), s in zip(blocks, scale):
+        assert np.abs(ng[lo:hi] - ref[0][lo:hi]).max() <= 3.0 * spread[kind] * s, (lo, spread)
     if not rotation:
         assert np.all(ng[18:] == 0.0)
