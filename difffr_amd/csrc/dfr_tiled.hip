@@ -877,9 +877,9 @@ k_expand_lists(GridDesc g, const uint32_t* __restrict__ fstart, int nf, const ui
 
 // Copies a step's lists to another set of buffers: the rows and map entries in
 // use, which is all that a pass reads.  A thread per particle, a workgroup per
-// brick for the maps; bound by memory.  Whole buffers hold 64 fluid slots and
-// maxb boundary samples a particle and 2,560 map entries a brick, some 500 MB at
-// 1M particles; the entries in use take 40 us there (250,000: 14.5), and a pass of
+// brick for the maps; bound by memory.  Whole buffers hold 128 fluid slots (2 bytes)
+// and maxb boundary samples (4) a particle and 2,560 map entries a brick, some 570 MB
+// at 1M particles; the entries in use take 40 us there (250,000: 14.5), and a pass of
 // four recorded steps with their reverse went from 8454 to 8284 us (six
 // checkpointed ones at 250,000: 8167 to 8076).
 __global__ void __launch_bounds__(DFR_BLOCK)
