@@ -142,11 +142,12 @@ __global__ void __launch_bounds__(DFR_BLOCK) k_scan_sums(SortSets S, uint32_t m)
   if (threadIdx.x == 0) sums[m] = carry;
 }
 
-__global__ void __launch_bounds__(DFR_BLOCK) k_scan_add(SortSets S, uint32_t n, int summed) {
+template <bool SUMMED>
+__global__ void __launch_bounds__(DFR_BLOCK) k_scan_add(SortSets S, uint32_t n) {
   const SortSet& T = S.s[blockIdx.y];
   __shared__ uint32_t lds[DFR_BLOCK / 64 + 1];
   uint32_t add, end;
-  if (summed) {
+  if constexpr (SUMMED) {
     add = T.tile_sums[blockIdx.x];
     end = T.tile_sums[blockIdx.x + 1];
   } else {
@@ -250,7 +251,7 @@ static void launch_sort_sets(const SortSets& S, int nsets, const FluidMove& M, c
   hipLaunchKernelGGL(k_scan_tiles, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk);
   const bool many = tiles > SCAN_SUMS_TILES;
   if (many) hipLaunchKernelGGL(k_scan_sums, dim3(nsets), dim3(DFR_BLOCK), 0, s, S, tiles);
-  hipLaunchKernelGGL(k_scan_add, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk, (int)many);
+  hipLaunchKernelGGL(many ? k_scan_add<true> : k_scan_add<false>, dim3(tiles, nsets), dim3(DFR_BLOCK), 0, s, S, nk);
   if (particle_blocks) {
     hipLaunchKernelGGL(k_scatter, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S);
     hipLaunchKernelGGL(k_place, dim3(particle_blocks), dim3(DFR_BLOCK), 0, s, S, M);
