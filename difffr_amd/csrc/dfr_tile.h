@@ -338,6 +338,24 @@ __device__ inline void for_fluid_terms(const uint4* __restrict__ nbr8, size_t st
   }
 }
 
+// The same order with the particles read from global memory (a halo beyond the LDS
+// capacity): four slots a round, lane l of the quad takes the l-th, one pair a lane in
+// flight (two spill a register of the velocity update).
+template <class Load, class Term, class Acc>
+__device__ inline void for_fluid_terms_rolled(const uint4* __restrict__ nbr8, size_t stride, uint32_t i, uint32_t nF,
+                                              int l, Load&& load, Term&& term, Acc&& acc) {
+  const uint16_t* __restrict__ slots = reinterpret_cast<const uint16_t*>(nbr8);
+#pragma unroll 1
+  for (uint32_t k0 = 0; k0 < nF; k0 += 4) {
+    const uint32_t k = k0 + (uint32_t)l;  // of the same pack as k0; past the list's end a pack holds slot 0
+    const auto t = term(load((uint32_t)slots[((size_t)(k / PACK) * stride + i) * PACK + k % PACK]), k < nF);
+    acc(quad_bcast<0>(t));
+    acc(quad_bcast<1>(t));
+    acc(quad_bcast<2>(t));
+    acc(quad_bcast<3>(t));
+  }
+}
+
 // Which product of a boundary pair's three is rounded by itself, and whether its
 // share is added fused, has always gone by the neighbour's place u in its group
 // of the one-lane loop; both forms take it from u, so that a particle's sums are

@@ -678,8 +678,8 @@ k_velocity_update_t(PassArgs a, const float* __restrict__ kfield, float* __restr
           q.w = kfield[j];
           return q;
         };
-        for_fluid_terms<2, L>(a.nbr8, stride, i, nF, l, far,
-                              [&](const float4& q, bool live) { return pair(q.x, q.y, q.z, q.w, live); }, add);
+        for_fluid_terms_rolled(a.nbr8, stride, i, nF, l, far,
+                               [&](const float4& q, bool live) { return pair(q.x, q.y, q.z, q.w, live); }, add);
       }
       {
         const float dv = c.dt * c.V_f;
@@ -821,7 +821,7 @@ k_recompute_t(PassArgs a, int mode, float kcoef, const float* __restrict__ rho, 
         const float4 q = a.pos[j], v = a.vel[j];
         return Slot6{make_float4(q.x, q.y, q.z, v.x), make_float2(v.y, v.z)};
       };
-      for_fluid_terms<4, L>(a.nbr8, stride, i, nF, l, far, [&](const Slot6& q, bool live) {
+      for_fluid_terms_rolled(a.nbr8, stride, i, nF, l, far, [&](const Slot6& q, bool live) {
         return pair(q.a.x, q.a.y, q.a.z, q.a.w, q.b.x, q.b.y, live);
       }, add);
     }
