@@ -390,7 +390,7 @@ uint32_t filled_bricks(const GridDesc& g, const std::vector<float>& x, int64_t n
   for (int64_t i = 0; i < n; ++i) {
     size_t b[3];
     for (int k = 0; k < 3; ++k)
-      b[k] = (size_t)std::min(std::max((int)((x[3 * i + k] - g.lo[k]) * g.inv_cs), 0), g.n[k] - 1) / 4;
+      b[k] = (size_t)std::fmin(std::fmax((x[3 * i + k] - g.lo[k]) * g.inv_cs, 0.f), (float)(g.n[k] - 1)) / 4;
     const size_t at = (b[2] * g.bn[1] + b[1]) * g.bn[0] + b[0];
     filled += seen[at] ? 0u : 1u;
     seen[at] = true;
